@@ -4,6 +4,7 @@
 #include "lira_internal.hpp"
 
 #include <cmath>
+#include <memory>
 
 namespace lira {
 
@@ -199,7 +200,9 @@ void moment_coefficients(double *coef) {
                     }
                 }
     };
-    static Poly cr[E][E], ci[E][E];
+    // on the heap, one set per call: solvers on several threads build their tables at the same time
+    const std::unique_ptr<Poly[][E]> cr_mem(new Poly[E][E]), ci_mem(new Poly[E][E]);
+    Poly(*cr)[E] = cr_mem.get(), (*ci)[E] = ci_mem.get();
     for (int l = 0; l < E; l++)
         for (int m = 0; m < E; m++) {
             zero(cr[l][m]);
@@ -228,7 +231,7 @@ void moment_coefficients(double *coef) {
             const double bq = std::sqrt(tt > 0.0 ? tt : 0.0);
             const double d = std::sqrt(lf * lf - mf * mf);
             for (int part = 0; part < 2; part++) {
-                Poly(&C)[E][E] = part == 0 ? cr : ci;
+                Poly(*C)[E] = part == 0 ? cr : ci;
                 times(C[l - 1][m], 2, t1);
                 zero(t2);
                 if (l >= 2 && m <= l - 2) times(C[l - 2][m], 3, t2);
