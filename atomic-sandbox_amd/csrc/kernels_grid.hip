@@ -29,10 +29,9 @@ void DevBuf::release() {
     bytes = 0;
 }
 
-// 8th-order second-derivative coefficients c1..c4 (qm/src/stencil.rs:24; c0 = -205/72 is folded into the
-// differences: sum_m c_m[(f+ - f) + (f- - f)] per axis equals c0 f + sum_m c_m (f+ + f-) since c0 = -2 sum c_m).
-// Kernels use them as T(Cm): an f32 stencil computes in f32 throughout (a bare double constant would promote every
-// tap product to f64).
+// 8th-order second-derivative coefficients c1..c4 (qm/src/stencil.rs:24), c0 = -205/72 = -2 sum c_m. The kernels use
+// their partial sums in their own precision (StK below): a bare double constant would promote an f32 stencil's products
+// to f64.
 #define C1 (8.0 / 5.0)
 #define C2 (-1.0 / 5.0)
 #define C3 (8.0 / 315.0)
@@ -73,16 +72,21 @@ template <> __device__ __forceinline__ void bstore_nt<double>(double v, BufRes r
 }
 
 // ------------------------------------------------------------------------------------------ stencil ----
-// 2.5-D z-streaming: a workgroup owns a TX x TY tile of (x, y) columns of one band and a chunk of z planes, TX = 64
-// (one wave per row) or 32 (a wave covers two rows: for n just above a multiple of 32, e.g. 95 = 3 x 32 - 1, the 64-wide
-// tile would leave a quarter of its lanes outside the box). Each thread keeps its RPT columns' 9-plane z-window in
-// registers; the x/y taps of the current plane come from an LDS tile with a 4-point halo (double-buffered: one barrier
-// per plane). The potential V is read once per point.
-
-// Register state of one thread: the 9-plane z window of its RPT columns (plane p in slot (p - z0 + 4) mod 9) and the
-// look-ahead queues of its halo cells, V and R (plane p in slot (p - z0) mod 3). The z loop is unrolled by 9 so every
-// slot index is a compile-time constant: registers rotate by name and are never copied, so a look-ahead load is only
-// waited for when its plane is used.
+// 2.5-D z-streaming: a workgroup owns a TX x TYL tile of (x, y) columns of one band and a chunk of z planes; a lane
+// owns VX consecutive x points of one row (16 bytes: float4 / double2) and streams them along z. The z neighbours stay
+// in registers, the x / y neighbours of the current plane come from a double-buffered LDS tile with a 4-point halo (one
+// barrier per plane).
+//
+// The second derivative along an axis is taken from first differences D_j = f_{j+1} - f_j:
+//   sum_m c_m (f_m - 2 f_0 + f_{-m}) = sum_{j=0..3} K_j (D_j - D_{-1-j}),  K_j = sum_{m>j} c_m.
+// A difference of neighbouring values of a smooth field is exact or nearly so in its own precision, and the sum of
+// second differences never carries the large central term, so the f32 stencil keeps its accuracy (2-norm error of H.X
+// against 64 bits on orbital-like bands, 95^3: 6e-8 .. 8e-8). Neighbouring outputs share their D's: along z they stay in
+// registers (four below the plane, four of the planes ahead), along x a lane's VX points share VX + 7, and each axis costs 8 more operations per
+// point: 41 VALU operations per f32 point, against 56 of the pair form c_m [(f_m - f_0) + (f_{-m} - f_0)] that this
+// replaces. Without packed FP32 instructions an f32 operation issues at the f64 rate (39 T lane-operations/s), so at
+// 192^3 x 64 the pair form alone cost 0.65 ms of VALU issue against 0.63 ms for the bytes at the copy rate.
+//
 // XCD-aware workgroup order. The dispatcher hands consecutive workgroup ids to the 8 XCDs round-robin (id mod 8);
 // each XCD has its own L2. The stencil launches a 1-D grid and gives XCD x the contiguous logical range
 // [x P, (x + 1) P) of (band, z chunk, tile) work items, tiles fastest: the tiles of one band (whose halos overlap) and
@@ -144,660 +148,322 @@ template <int W> struct PlaneUnroll<W, W> {
     template <typename F> __device__ __forceinline__ static void run(F &) {}
 };
 
-// The z window holds W >= 9 planes: the 9 the 8th-order z taps of the current plane z read (z - 4 .. z + 4) and
-// W - 9 planes of look-ahead, so the plane a step loads (z + W - 5, into the slot plane z - 5 frees) is first used
-// W - 9 steps later. W is a multiple of 3, the length of the halo / V / R queues (loaded two planes ahead).
-template <typename T, int RPT, int W> struct StRegs {
-    T q[W][RPT];
-    T hq[3][3];
-    T vq[3][RPT];
-    T rq[3][RPT];
-};
-
-template <typename T, int RPT> struct StCtx {
-    BufRes bx, bo, bv, br;  // x and out of this band, V, R of this band
-    unsigned pb;            // bytes per plane
-    unsigned co[RPT];       // this lane's centre rows (gx, y0 + ty + (256 / TX) rr): byte offsets in a plane, or BUF_OOB
-    unsigned ho0, ho1, hox; // its y-halo cells (gx, y0 - 4 + hly0 / hly1; hly1 only at TX = 64) and x-halo cell
-    int n;
-    int gx, x0, y0, tx, ty;
-    int hly0, hly1, hxr, hlx;
-    bool has_xh;
-    T inv_h2, scale, omega, diag_t, lamb;
-    __device__ T ld(BufRes r, unsigned off, int zz) const { return bload<T>(r, off + (unsigned)zz * pb); }
-};
-
-template <typename T, int MODE, int RPT, int W, int TX, int SLOT>
-__device__ __forceinline__ void st_side(StRegs<T, RPT, W> &R, const StCtx<T, RPT> &c, int zz) {
-    constexpr int QS = SLOT % 3;
-    R.hq[QS][0] = c.ld(c.bx, c.ho0, zz);
-    if (TX == 64) R.hq[QS][1] = c.ld(c.bx, c.ho1, zz);
-    R.hq[QS][2] = c.ld(c.bx, c.hox, zz);
-#pragma unroll
-    for (int rr = 0; rr < RPT; rr++) {
-        if (MODE != ST_LAP) R.vq[QS][rr] = c.ld(c.bv, c.co[rr], zz);
-        if (MODE == ST_JAC) R.rq[QS][rr] = c.ld(c.br, c.co[rr], zz);
-    }
-}
-
-// one plane z of the stream; S = (z - z0) mod W
-template <typename T, int MODE, int RPT, int W, int TX, int S>
-__device__ __forceinline__ void st_plane(StRegs<T, RPT, W> &R, const StCtx<T, RPT> &c,
-                                         T (*tile)[(256 / TX) * RPT + 8][TX + 8], int z, int buf) {
-    constexpr int TYB = 256 / TX;  // rows per pass of the workgroup
-    constexpr int C0 = (S + 4) % W;
-    constexpr int NEW = (S + W - 1) % W;
-    constexpr int HS = S % 3;
-#pragma unroll
-    for (int rr = 0; rr < RPT; rr++) R.q[NEW][rr] = c.ld(c.bx, c.co[rr], z + W - 5);
-    st_side<T, MODE, RPT, W, TX, S + 2>(R, c, z + 2);
-    T(*tl)[TX + 8] = tile[buf];
-#pragma unroll
-    for (int rr = 0; rr < RPT; rr++) tl[c.ty + TYB * rr + 4][c.tx + 4] = R.q[C0][rr];
-    tl[c.hly0][c.tx + 4] = R.hq[HS][0];
-    if (TX == 64) tl[c.hly1][c.tx + 4] = R.hq[HS][1];
-    if (c.has_xh) tl[c.hxr][c.hlx] = R.hq[HS][2];
-    __syncthreads();
-#pragma unroll
-    for (int rr = 0; rr < RPT; rr++) {
-        const int ly = c.ty + TYB * rr + 4, lx = c.tx + 4;
-        const T ce = R.q[C0][rr];
-        T ax = T(C1) * ((tl[ly][lx + 1] - ce) + (tl[ly][lx - 1] - ce)) + T(C2) * ((tl[ly][lx + 2] - ce) + (tl[ly][lx - 2] - ce)) +
-               T(C3) * ((tl[ly][lx + 3] - ce) + (tl[ly][lx - 3] - ce)) + T(C4) * ((tl[ly][lx + 4] - ce) + (tl[ly][lx - 4] - ce));
-        T ay = T(C1) * ((tl[ly + 1][lx] - ce) + (tl[ly - 1][lx] - ce)) + T(C2) * ((tl[ly + 2][lx] - ce) + (tl[ly - 2][lx] - ce)) +
-               T(C3) * ((tl[ly + 3][lx] - ce) + (tl[ly - 3][lx] - ce)) + T(C4) * ((tl[ly + 4][lx] - ce) + (tl[ly - 4][lx] - ce));
-        T az = T(C1) * ((R.q[(S + 5) % W][rr] - ce) + (R.q[(S + 3) % W][rr] - ce)) +
-               T(C2) * ((R.q[(S + 6) % W][rr] - ce) + (R.q[(S + 2) % W][rr] - ce)) +
-               T(C3) * ((R.q[(S + 7) % W][rr] - ce) + (R.q[(S + 1) % W][rr] - ce)) +
-               T(C4) * ((R.q[(S + 8) % W][rr] - ce) + (R.q[S % W][rr] - ce));
-        const T lap = ((ax + ay) + az) * c.inv_h2;
-        T o;
-        if (MODE == ST_LAP) {
-            o = c.scale * lap;
-        } else if (MODE == ST_HAM) {
-            o = T(-0.5) * lap + R.vq[HS][rr] * ce;
-        } else {
-            const T vv = R.vq[HS][rr];
-            const T hw = T(-0.5) * lap + vv * ce - c.lamb * ce;
-            T d = c.diag_t + vv - c.lamb;
-            d = d > T(0.1) ? d : T(0.1);
-            o = ce + c.omega / d * (R.rq[HS][rr] - hw);
-        }
-        // a row outside the box has offset BUF_OOB: its store is dropped
-        bstore_nt<T>(o, c.bo, c.co[rr] + (unsigned)z * c.pb);
-    }
-}
-
-template <typename T, int MODE, int RPT, int W, int TX>
-__global__ __launch_bounds__(256) void k_stencil(const T *__restrict__ x, T *__restrict__ out, const T *__restrict__ v,
-                                                 const T *__restrict__ r, const double *__restrict__ lam, int n,
-                                                 long N, int zc, int nb, int order, T inv_h2, T scale, T omega,
-                                                 T diag_t, const T *__restrict__ x2, T *__restrict__ out2, int nb1) {
-    static_assert(TX == 64 || TX == 32, "tile width");
-    constexpr int TYB = 256 / TX;  // workgroup (TX, TYB)
-    constexpr int TY = TYB * RPT;
-    // the y halo (8 rows of TX cells) takes 512 / TX cells per lane, the x halo (TY + 8 rows of 8 cells) one
-    static_assert(8 * (TY + 8) <= 256, "x halo larger than the workgroup");
-    __shared__ T tile[2][TY + 8][TX + 8];
-    StCtx<T, RPT> c;
-    c.tx = threadIdx.x;
-    c.ty = threadIdx.y;
-    const int t = c.ty * TX + c.tx;
-    const int nzc = (n + zc - 1) / zc;
-    const StWork wk = st_decode((n + TX - 1) / TX, (n + TY - 1) / TY, nzc, nb, order);
-    if (!wk.valid) return;
-    c.x0 = wk.tile_x * TX;
-    c.y0 = wk.tile_y * TY;
-    const int band = wk.band;
-    const int z0 = wk.zchunk * zc;
-    const int z1 = min(n, z0 + zc);
-    const long fb = N * (long)sizeof(T);
-    c.bx = field_res(band < nb1 ? x + (long)band * N : x2 + (long)(band - nb1) * N, fb);
-    c.bo = field_res(band < nb1 ? out + (long)band * N : out2 + (long)(band - nb1) * N, fb);
-    c.bv = field_res(v, MODE == ST_LAP ? 0 : fb);
-    c.br = field_res(MODE == ST_JAC ? r + (long)band * N : x, MODE == ST_JAC ? fb : 0);
-    c.lamb = MODE == ST_JAC ? (T)lam[band] : T(0);
-    c.n = n;
-    c.pb = (unsigned)((long)n * n * (long)sizeof(T));
-    c.gx = c.x0 + c.tx;
-#pragma unroll
-    for (int rr = 0; rr < RPT; rr++) c.co[rr] = row_off(c.gx, c.y0 + c.ty + TYB * rr, n, (int)sizeof(T));
-    // y-halo rows 0..3 above the tile, 4..7 below it (LDS rows TY + 4 ..): row ty, and at TX = 64 also row ty + 4
-    const int hy0 = c.ty, hy1 = c.ty + 4;
-    c.hly0 = hy0 < 4 ? hy0 : TY + hy0;
-    c.hly1 = TY + hy1;
-    c.has_xh = t < 8 * (TY + 8);
-    c.hxr = t >> 3;
-    const int hxc = t & 7;
-    c.hlx = hxc < 4 ? hxc : TX + hxc;
-    c.ho0 = row_off(c.gx, c.y0 - 4 + c.hly0, n, (int)sizeof(T));
-    c.ho1 = TX == 64 ? row_off(c.gx, c.y0 - 4 + c.hly1, n, (int)sizeof(T)) : BUF_OOB;
-    c.hox = c.has_xh ? row_off(c.x0 - 4 + c.hlx, c.y0 - 4 + c.hxr, n, (int)sizeof(T)) : BUF_OOB;
-    c.inv_h2 = inv_h2;
-    c.scale = scale;
-    c.omega = omega;
-    c.diag_t = diag_t;
-
-    StRegs<T, RPT, W> R;
-#pragma unroll
-    for (int d = 0; d < W - 1; d++)
-#pragma unroll
-        for (int rr = 0; rr < RPT; rr++) R.q[d][rr] = c.ld(c.bx, c.co[rr], z0 - 4 + d);
-    st_side<T, MODE, RPT, W, TX, 0>(R, c, z0);
-    st_side<T, MODE, RPT, W, TX, 1>(R, c, z0 + 1);
-
-    // consecutive planes alternate the two LDS buffers (plane p uses buffer (p - z0) & 1): one barrier per plane then
-    // separates every write of a buffer from the previous reads of it
-    int z = z0;
-    for (; z + W <= z1; z += W) {
-        const int b = (z - z0) & 1;
-        auto step = [&](auto sc) {
-            constexpr int S = decltype(sc)::value;
-            st_plane<T, MODE, RPT, W, TX, S>(R, c, tile, z + S, b ^ (S & 1));
-        };
-        PlaneUnroll<0, W>::run(step);
-    }
-    // remainder (< W planes) with the same slot sequence
-    const int b = (z - z0) & 1;
-    auto tail = [&](auto sc) {
-        constexpr int S = decltype(sc)::value;
-        if (z + S < z1) st_plane<T, MODE, RPT, W, TX, S>(R, c, tile, z + S, b ^ (S & 1));
-    };
-    PlaneUnroll<0, W - 1>::run(tail);
-}
-
-// ---- vectorised stencil: each lane owns VX consecutive x points (16-byte loads and stores: float4 / double2) ----
-// Requires n % VX == 0 so every vector is aligned and lies wholly inside or outside the box. Workgroup 16 x 16 lanes:
-// tile TX = 16 VX columns x TY = 16 RPT rows (row ty + 16 rr). z window, halo/V/R look-ahead and LDS double buffering
-// as the scalar kernel; x taps are read from LDS as three 16-byte vectors, y taps as one vector per row.
+// native 16-byte vectors: VX = 4 f32 or 2 f64 points
 template <typename T> struct Vec16;
 template <> struct Vec16<float> {
-    typedef float4 type;
+    typedef float type __attribute__((ext_vector_type(4)));
     static constexpr int N = 4;
 };
 template <> struct Vec16<double> {
-    typedef double2 type;
+    typedef double type __attribute__((ext_vector_type(2)));
     static constexpr int N = 2;
 };
+// 16-byte buffer load / nontemporal store of one vector at any element alignment; the range check is per dword
+template <typename T> __device__ __forceinline__ typename Vec16<T>::type bloadv(BufRes r, unsigned off) {
+    return __builtin_bit_cast(typename Vec16<T>::type, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+}
+template <typename V> __device__ __forceinline__ void bstorev_nt(V v, BufRes r, unsigned off) {
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, off, 0, 2);
+}
 
-template <typename T, int RPT, int W> struct SvRegs {
-    typedef typename Vec16<T>::type V;
-    V q[W][RPT];
-    V hq[3];
-    V hq2[3];  // second x-halo vector when a vector holds fewer than the 4 halo points (double2)
-    V vq[3][RPT];
-    V rq[3][RPT];
+constexpr int ST_AHEAD = 6;  // a lane loads its plane z + ST_AHEAD at plane z
+// K_j = sum_{m > j} c_m. Rounded to f32 one by one they would scale every Laplacian by 1 + 5.3e-8 (sum (2j + 1) K_j, K_0's
+// rounding); the f32 set takes the neighbouring values (2, 4 and 8 units in the last place off) that keep that sum within
+// 6e-9 of 1 and the 4th moment within 6e-8 of 0.
+template <typename T> struct StK;
+template <> struct StK<double> {
+    static constexpr double k[4] = {C1 + C2 + C3 + C4, C2 + C3 + C4, C3 + C4, C4};
+};
+template <> struct StK<float> {
+    static constexpr float k[4] = {1.4236111640930176f, -0.1763889193534851f, 0.023611119017004967f,
+                                   -0.0017857152270153165f};
 };
 
-// native 16-byte vectors for the buffer intrinsics
-typedef float lira_nf4 __attribute__((ext_vector_type(4)));
-typedef double lira_nd2 __attribute__((ext_vector_type(2)));
-
-template <typename T> __device__ __forceinline__ T vget(const typename Vec16<T>::type &v, int i);
-template <> __device__ __forceinline__ float vget<float>(const float4 &v, int i) {
-    return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
-}
-template <> __device__ __forceinline__ double vget<double>(const double2 &v, int i) { return i == 0 ? v.x : v.y; }
-template <typename T> __device__ __forceinline__ void vset(typename Vec16<T>::type &v, int i, T x);
-template <> __device__ __forceinline__ void vset<float>(float4 &v, int i, float x) {
-    if (i == 0) v.x = x; else if (i == 1) v.y = x; else if (i == 2) v.z = x; else v.w = x;
-}
-template <> __device__ __forceinline__ void vset<double>(double2 &v, int i, double x) {
-    if (i == 0) v.x = x; else v.y = x;
-}
-// 16-byte buffer load / nontemporal store of one vector (float4 or double2)
-template <typename T> __device__ __forceinline__ typename Vec16<T>::type bloadv(BufRes r, unsigned off);
-template <> __device__ __forceinline__ float4 bloadv<float>(BufRes r, unsigned off) {
-    const lira_nf4 t = __builtin_bit_cast(lira_nf4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
-    return make_float4(t.x, t.y, t.z, t.w);
-}
-template <> __device__ __forceinline__ double2 bloadv<double>(BufRes r, unsigned off) {
-    const lira_nd2 t = __builtin_bit_cast(lira_nd2, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
-    return make_double2(t.x, t.y);
-}
-__device__ __forceinline__ void bstorev_nt(const float4 &v, BufRes r, unsigned off) {
-    typedef unsigned u4 __attribute__((ext_vector_type(4)));
-    const lira_nf4 t = {v.x, v.y, v.z, v.w};
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, t), r, off, 0, 2);
-}
-__device__ __forceinline__ void bstorev_nt(const double2 &v, BufRes r, unsigned off) {
-    typedef unsigned u4 __attribute__((ext_vector_type(4)));
-    const lira_nd2 t = {v.x, v.y};
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, t), r, off, 0, 2);
-}
-
-template <typename T, int RPT> struct SvCtx {
+// Register state of a lane: F holds its vector on planes z .. z + 5 (plane p in slot (p - z0) mod 8; step z loads plane
+// z + 6), D the differences D_{z-4} .. D_{z-1} (D_j in slot (j - z0) mod 4; step z replaces D_{z-4} by D_z), and hq /
+// vq / rq its halo vectors, V and R, loaded two planes ahead. The z loop is unrolled by 8 so every slot is a compile-time
+// constant: registers rotate by name, and a load is only waited for when its plane is used. Keeping D_z .. D_{z+3} as
+// well would save three operations per point but 16 registers: at three waves per SIMD (168 registers) the Jacobi sweep
+// then spills (95^3 x 8 f32: 24.9 us, 19.6 us without them).
+template <typename T, int HV> struct StRegs {
     typedef typename Vec16<T>::type V;
-    static constexpr int VX = Vec16<T>::N;
-    BufRes bx, bo, bv, br;
-    unsigned pb;                // bytes per plane
-    unsigned co[RPT];           // centre rows (gx, y0 + ty + 16 rr): byte offsets in a plane, or BUF_OOB
-    unsigned ho, ho2;           // this lane's halo vector(s), or BUF_OOB
-    int n;
-    int x0, y0, tx, ty, gx;
-    int h_ly, h_lx;             // this lane's halo vector (LDS row/col), if any
-    bool has_h, has_h2;         // has_h2: an x-halo lane that also loads the vector at h_gx + VX
-    T inv_h2, scale, omega, diag_t, lamb;
-    __device__ V ldv(BufRes r, unsigned off, int zz) const { return bloadv<T>(r, off + (unsigned)zz * pb); }
+    V F[8], D[4];
+    V hq[2][HV];
+    V vq[2], rq[2];
 };
 
-template <typename T, int MODE, int RPT, int W, int SLOT>
-__device__ __forceinline__ void sv_side(SvRegs<T, RPT, W> &R, const SvCtx<T, RPT> &c, int zz) {
-    constexpr int QS = SLOT % 3;
-    R.hq[QS] = c.ldv(c.bx, c.ho, zz);
-    if (SvCtx<T, RPT>::VX < 4) R.hq2[QS] = c.ldv(c.bx, c.ho2, zz);
-#pragma unroll
-    for (int rr = 0; rr < RPT; rr++) {
-        if (MODE != ST_LAP) R.vq[QS][rr] = c.ldv(c.bv, c.co[rr], zz);
-        if (MODE == ST_JAC) R.rq[QS][rr] = c.ldv(c.br, c.co[rr], zz);
+template <typename T, int HV> struct StCtx {
+    typedef typename Vec16<T>::type V;
+    BufRes bx, bo, bv, br;  // x and out of this band, V, R of this band
+    unsigned pb;            // bytes per plane
+    unsigned co;            // this lane's vector: byte offset in a plane, or BUF_OOB
+    unsigned ho[HV];        // its halo vectors, or BUF_OOB
+    int hl[HV];             // their element offset in an LDS plane, -1: none
+    int hnv[HV];            // points of them inside the box (the rest belong to the next row)
+    int nv;                 // points of the lane's vector inside the box
+    int lo;                 // the lane's element offset in an LDS plane
+    int n, zlim;            // planes at or past zlim are not loaded
+    T hs, omega, diag_t, lamb;
+    // plane zz at byte offset off; a plane past the last one the chunk needs reads plane n: out of range, 0
+    __device__ V ld(BufRes r, unsigned off, int zz, int lim) const {
+        return bloadv<T>(r, off + (unsigned)(zz < lim ? zz : n) * pb);
     }
+};
+
+template <typename V, int VX> __device__ __forceinline__ V st_mask(V v, int nv) {
+#pragma unroll
+    for (int i = 0; i < VX; i++) v[i] = i < nv ? v[i] : 0;
+    return v;
 }
 
-template <typename T, int MODE, int RPT, int W, int S, int LXP>
-__device__ __forceinline__ void sv_plane(SvRegs<T, RPT, W> &R, const SvCtx<T, RPT> &c, T (*tile)[16 * RPT + 8][LXP],
-                                         int z, int buf) {
+// omega / d for d >= 0.1: a reciprocal estimate, the quotient and one residual correction
+__device__ __forceinline__ float st_quot(float a, float d) {
+    const float r = __builtin_amdgcn_rcpf(d), q = a * r;
+    return __builtin_fmaf(__builtin_fmaf(-d, q, a), r, q);
+}
+__device__ __forceinline__ double st_quot(double a, double d) { return a / d; }
+__device__ __forceinline__ float st_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double st_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// one plane z of the stream; S = (z - z0) mod 8
+template <typename T, int MODE, int TXL, int TYL, bool XT, bool RAG, int HV, int S>
+__device__ __forceinline__ void st_plane(StRegs<T, HV> &R, const StCtx<T, HV> &c, T *tl, int z, int z1) {
     typedef typename Vec16<T>::type V;
     constexpr int VX = Vec16<T>::N;
-    constexpr int C0 = (S + 4) % W;
-    constexpr int NEW = (S + W - 1) % W;
-    constexpr int HS = S % 3;
+    constexpr int LXP = TXL * VX + 8;
+    R.F[(S + ST_AHEAD) & 7] = c.ld(c.bx, c.co, z + ST_AHEAD, c.zlim);
+    const V ce = RAG ? st_mask<V, VX>(R.F[S], c.nv) : R.F[S];
+    *reinterpret_cast<V *>(tl + c.lo) = ce;
 #pragma unroll
-    for (int rr = 0; rr < RPT; rr++) R.q[NEW][rr] = c.ldv(c.bx, c.co[rr], z + W - 5);
-    sv_side<T, MODE, RPT, W, S + 2>(R, c, z + 2);
-    T(*tl)[LXP] = tile[buf];
-    const int lx = 4 + VX * c.tx;  // LDS column of this lane's first point
+    for (int k = 0; k < HV; k++)
+        if (c.hl[k] >= 0)
+            *reinterpret_cast<V *>(tl + c.hl[k]) = XT && RAG ? st_mask<V, VX>(R.hq[S & 1][k], c.hnv[k]) : R.hq[S & 1][k];
 #pragma unroll
-    for (int rr = 0; rr < RPT; rr++) *reinterpret_cast<V *>(&tl[c.ty + 16 * rr + 4][lx]) = R.q[C0][rr];
-    if (c.has_h) *reinterpret_cast<V *>(&tl[c.h_ly][c.h_lx]) = R.hq[HS];
-    if (VX < 4 && c.has_h2) *reinterpret_cast<V *>(&tl[c.h_ly][c.h_lx + VX]) = R.hq2[HS];
+    for (int k = 0; k < HV; k++) R.hq[S & 1][k] = c.ld(c.bx, c.ho[k], z + 2, z1);
     __syncthreads();
+    // The second differences e_j = D_j - D_{-1-j} of each axis: those of j = 3, 2, 1 (coefficients up to K0 / 8) go into acc
+    // as they come, the j = 0 ones are summed over the axes and added last, so the large partial sums are rounded three
+    // times in all.
+    V acc, e0;
+    auto add = [&](V e, T k) {
 #pragma unroll
-    for (int rr = 0; rr < RPT; rr++) {
-        const int ly = c.ty + 16 * rr + 4;
-        // x window: 4 + VX + 4 values starting at lx - 4
-        T w[VX + 8];
+        for (int i = 0; i < VX; i++) acc[i] = st_fma(e[i], k, acc[i]);
+    };
+    // z
+    {
+        V dn[4];
 #pragma unroll
-        for (int b = 0; b < (VX + 8) / VX; b++) {
-            const V vv = *reinterpret_cast<const V *>(&tl[ly][lx - 4 + VX * b]);
+        for (int j = 0; j < 4; j++) dn[j] = R.F[(S + j + 1) & 7] - R.F[(S + j) & 7];
+        acc = (dn[3] - R.D[S & 3]) * StK<T>::k[3];
+        add(dn[2] - R.D[(S + 1) & 3], StK<T>::k[2]);
+        add(dn[1] - R.D[(S + 2) & 3], StK<T>::k[1]);
+        e0 = dn[0] - R.D[(S + 3) & 3];
+        R.D[S & 3] = dn[0];
+    }
+    // y: the eight rows about this one
+    {
+        V m[5], p[5];
+        m[0] = p[0] = ce;
 #pragma unroll
-            for (int i = 0; i < VX; i++) w[VX * b + i] = vget<T>(vv, i);
+        for (int q = 1; q <= 4; q++) {
+            m[q] = *reinterpret_cast<const V *>(tl + c.lo - q * LXP);
+            p[q] = *reinterpret_cast<const V *>(tl + c.lo + q * LXP);
         }
-        V ym[4], yp[4];
+        add((p[4] - p[3]) - (m[3] - m[4]), StK<T>::k[3]);
+        add((p[3] - p[2]) - (m[2] - m[3]), StK<T>::k[2]);
+        add((p[2] - p[1]) - (m[1] - m[2]), StK<T>::k[1]);
+        e0 += (p[1] - p[0]) - (m[0] - m[1]);
+    }
+    // x: the VX + 8 points of this row about the lane's, their differences shared by its points
+    {
+        T w[VX + 8], d[VX + 7];
 #pragma unroll
-        for (int m = 1; m <= 4; m++) {
-            ym[m - 1] = *reinterpret_cast<const V *>(&tl[ly - m][lx]);
-            yp[m - 1] = *reinterpret_cast<const V *>(&tl[ly + m][lx]);
-        }
-        V outv;
+        for (int b = 0; b < 4 / VX; b++) {
+            const V l = *reinterpret_cast<const V *>(tl + c.lo - 4 + VX * b);
+            const V r = *reinterpret_cast<const V *>(tl + c.lo + VX + VX * b);
 #pragma unroll
-        for (int i = 0; i < VX; i++) {
-            const T ce = w[4 + i];
-            const T ax = T(C1) * ((w[5 + i] - ce) + (w[3 + i] - ce)) + T(C2) * ((w[6 + i] - ce) + (w[2 + i] - ce)) +
-                         T(C3) * ((w[7 + i] - ce) + (w[1 + i] - ce)) + T(C4) * ((w[8 + i] - ce) + (w[0 + i] - ce));
-            const T ay = T(C1) * ((vget<T>(yp[0], i) - ce) + (vget<T>(ym[0], i) - ce)) +
-                         T(C2) * ((vget<T>(yp[1], i) - ce) + (vget<T>(ym[1], i) - ce)) +
-                         T(C3) * ((vget<T>(yp[2], i) - ce) + (vget<T>(ym[2], i) - ce)) +
-                         T(C4) * ((vget<T>(yp[3], i) - ce) + (vget<T>(ym[3], i) - ce));
-            const T az = T(C1) * ((vget<T>(R.q[(S + 5) % W][rr], i) - ce) + (vget<T>(R.q[(S + 3) % W][rr], i) - ce)) +
-                         T(C2) * ((vget<T>(R.q[(S + 6) % W][rr], i) - ce) + (vget<T>(R.q[(S + 2) % W][rr], i) - ce)) +
-                         T(C3) * ((vget<T>(R.q[(S + 7) % W][rr], i) - ce) + (vget<T>(R.q[(S + 1) % W][rr], i) - ce)) +
-                         T(C4) * ((vget<T>(R.q[(S + 8) % W][rr], i) - ce) + (vget<T>(R.q[S % W][rr], i) - ce));
-            const T lap = ((ax + ay) + az) * c.inv_h2;
-            T o;
-            if (MODE == ST_LAP) {
-                o = c.scale * lap;
-            } else if (MODE == ST_HAM) {
-                o = T(-0.5) * lap + vget<T>(R.vq[HS][rr], i) * ce;
-            } else {
-                const T vv = vget<T>(R.vq[HS][rr], i);
-                const T hw = T(-0.5) * lap + vv * ce - c.lamb * ce;
-                T d = c.diag_t + vv - c.lamb;
-                d = d > T(0.1) ? d : T(0.1);
-                o = ce + c.omega / d * (vget<T>(R.rq[HS][rr], i) - hw);
+            for (int i = 0; i < VX; i++) {
+                w[VX * b + i] = l[i];
+                w[4 + VX + VX * b + i] = r[i];
             }
-            vset<T>(outv, i, o);
         }
-        // a row or vector outside the box has offset BUF_OOB: its store is dropped
-        bstorev_nt(outv, c.bo, c.co[rr] + (unsigned)z * c.pb);
+#pragma unroll
+        for (int i = 0; i < VX; i++) w[4 + i] = ce[i];
+#pragma unroll
+        for (int i = 0; i < VX + 7; i++) d[i] = w[i + 1] - w[i];
+#pragma unroll
+        for (int j = 3; j >= 1; j--)
+#pragma unroll
+            for (int i = 0; i < VX; i++) acc[i] = st_fma(d[4 + i + j] - d[3 + i - j], StK<T>::k[j], acc[i]);
+#pragma unroll
+        for (int i = 0; i < VX; i++) e0[i] += d[4 + i] - d[3 + i];
+    }
+    add(e0, StK<T>::k[0]);
+    V o;
+#pragma unroll
+    for (int i = 0; i < VX; i++) {
+        if (MODE == ST_LAP) {
+            o[i] = c.hs * acc[i];
+        } else if (MODE == ST_HAM) {
+            o[i] = st_fma(c.hs, acc[i], R.vq[S & 1][i] * ce[i]);
+        } else {
+            const T t = R.vq[S & 1][i] - c.lamb;
+            const T hw = st_fma(c.hs, acc[i], t * ce[i]);
+            T d = c.diag_t + t;
+            d = d > T(0.1) ? d : T(0.1);
+            o[i] = st_fma(st_quot(c.omega, d), R.rq[S & 1][i] - hw, ce[i]);
+        }
+    }
+    if (MODE != ST_LAP) R.vq[S & 1] = c.ld(c.bv, c.co, z + 2, z1);
+    if (MODE == ST_JAC) R.rq[S & 1] = c.ld(c.br, c.co, z + 2, z1);
+    // a lane outside the box has offset BUF_OOB: its store is dropped; the row's last vector may be partly inside
+    const unsigned so = c.co + (unsigned)z * c.pb;
+    if (!RAG || c.nv >= VX) {
+        bstorev_nt(o, c.bo, so);
+    } else {
+#pragma unroll
+        for (int i = 0; i < VX - 1; i++)
+            if (i < c.nv) bstore_nt<T>(o[i], c.bo, so + i * (unsigned)sizeof(T));
     }
 }
 
-template <typename T, int MODE, int RPT, int W>
-__global__ __launch_bounds__(256) void k_stencil_vec(const T *__restrict__ x, T *__restrict__ out,
-                                                     const T *__restrict__ v, const T *__restrict__ r,
-                                                     const double *__restrict__ lam, int n, long N, int zc, int nb,
-                                                     int order, T inv_h2, T scale, T omega, T diag_t,
-                                                     const T *__restrict__ x2, T *__restrict__ out2, int nb1) {
-    constexpr int VX = Vec16<T>::N;
-    constexpr int TX = 16 * VX, TY = 16 * RPT;
-    constexpr int LXP = TX + 8;
-    __shared__ __align__(16) T tile[2][TY + 8][LXP];
-    SvCtx<T, RPT> c;
-    c.tx = threadIdx.x;
-    c.ty = threadIdx.y;
-    const int t = c.ty * 16 + c.tx;
+// TXL lanes in x (TX = TXL VX columns), TYL rows. XT: several tiles in x (their x halos are loaded; with one tile the
+// x neighbours outside it are outside the box and its LDS halo columns stay 0). RAG: n is no multiple of VX, so a row's
+// last vector holds points of the next row, which are masked (as neighbours) and not stored.
+template <typename T, int MODE, int TXL, int TYL, bool XT, bool RAG>
+__global__ __launch_bounds__(TXL *TYL) __attribute__((amdgpu_waves_per_eu(3))) void k_stencil(const T *__restrict__ x, T *__restrict__ out,
+                                                      const T *__restrict__ v, const T *__restrict__ r,
+                                                      const double *__restrict__ lam, int n, long N, int zc, int nb,
+                                                      int order, T hs, T omega, T diag_t, const T *__restrict__ x2,
+                                                      T *__restrict__ out2, int nb1) {
+    typedef typename Vec16<T>::type V;
+    constexpr int VX = Vec16<T>::N, TX = TXL * VX, LXP = TX + 8, THREADS = TXL * TYL;
+    constexpr int XV = 4 / VX;  // x-halo vectors per row and side
+    constexpr int YH = 8 * TXL, XH = XT ? 2 * XV * TYL : 0, HV = (YH + XH + THREADS - 1) / THREADS;
+    static_assert(THREADS % 64 == 0, "whole waves");
+    __shared__ __align__(16) T tile[2][(TYL + 8) * LXP];
+    const int t = threadIdx.x, tx = t % TXL, ty = t / TXL;
     const int nzc = (n + zc - 1) / zc;
-    const StWork wk = st_decode((n + TX - 1) / TX, (n + TY - 1) / TY, nzc, nb, order);
+    const StWork wk = st_decode((n + TX - 1) / TX, (n + TYL - 1) / TYL, nzc, nb, order);
     if (!wk.valid) return;
-    c.x0 = wk.tile_x * TX;
-    c.y0 = wk.tile_y * TY;
-    const int band = wk.band;
-    const int z0 = wk.zchunk * zc;
-    const int z1 = min(n, z0 + zc);
+    const int x0 = wk.tile_x * TX, y0 = wk.tile_y * TYL, band = wk.band;
+    const int z0 = wk.zchunk * zc, z1 = min(n, z0 + zc);
     const long fb = N * (long)sizeof(T);
+    StCtx<T, HV> c;
     c.bx = field_res(band < nb1 ? x + (long)band * N : x2 + (long)(band - nb1) * N, fb);
     c.bo = field_res(band < nb1 ? out + (long)band * N : out2 + (long)(band - nb1) * N, fb);
-    c.bv = field_res(v, MODE == ST_LAP ? 0 : fb);
+    c.bv = field_res(MODE == ST_LAP ? x : v, MODE == ST_LAP ? 0 : fb);
     c.br = field_res(MODE == ST_JAC ? r + (long)band * N : x, MODE == ST_JAC ? fb : 0);
     c.lamb = MODE == ST_JAC ? (T)lam[band] : T(0);
     c.n = n;
+    c.zlim = z1 + 4;
     c.pb = (unsigned)((long)n * n * (long)sizeof(T));
-    c.gx = c.x0 + VX * c.tx;
-#pragma unroll
-    for (int rr = 0; rr < RPT; rr++) c.co[rr] = row_off(c.gx, c.y0 + c.ty + 16 * rr, n, (int)sizeof(T));
-    int h_gx = 0, h_gy = 0;
-    // halo vectors: 8 y-halo rows x 16 vectors (lanes 0..127), then (TY + 8) rows x 2 sides (lanes 128..); a side
-    // holds 4 points, i.e. 4 / VX vectors per x-halo lane
-    if (t < 128) {
-        const int row = t >> 4, col = t & 15;
-        c.h_ly = row < 4 ? row : TY + row;
-        c.h_lx = 4 + VX * col;
-        h_gx = c.x0 + VX * col;
-        h_gy = c.y0 - 4 + c.h_ly;
-        c.has_h = true;
-    } else if (t < 128 + 2 * (TY + 8)) {
-        const int e = t - 128, row = e >> 1, side = e & 1;
-        c.h_ly = row;
-        c.h_lx = side ? 4 + TX : 0;
-        h_gx = side ? c.x0 + TX : c.x0 - 4;
-        h_gy = c.y0 - 4 + row;
-        c.has_h = true;
-    } else {
-        c.h_ly = c.h_lx = 0;
-        c.has_h = false;
-    }
-    c.has_h2 = c.has_h && t >= 128;
-    c.ho = c.has_h ? row_off(h_gx, h_gy, n, (int)sizeof(T)) : BUF_OOB;
-    c.ho2 = c.has_h2 ? row_off(h_gx + VX, h_gy, n, (int)sizeof(T)) : BUF_OOB;
-    c.inv_h2 = inv_h2;
-    c.scale = scale;
+    const int gx = x0 + VX * tx;
+    c.co = row_off(gx, y0 + ty, n, (int)sizeof(T));
+    c.nv = n - gx;
+    c.lo = (ty + 4) * LXP + 4 + VX * tx;
+    c.hs = hs;
     c.omega = omega;
     c.diag_t = diag_t;
-    SvRegs<T, RPT, W> R;
+    // halo vectors: the 4 rows above and below the tile, then (XT) each row's 4 points left and right of it
 #pragma unroll
-    for (int d = 0; d < W - 1; d++)
+    for (int k = 0; k < HV; k++) {
+        const int e = t + k * THREADS;
+        int hgx = -1, hgy = -1;
+        c.hl[k] = -1;
+        if (e < YH) {
+            const int row = e / TXL, col = e % TXL, ly = row < 4 ? row : TYL + row;
+            hgx = x0 + VX * col;
+            hgy = y0 - 4 + ly;
+            c.hl[k] = ly * LXP + 4 + VX * col;
+        } else if (XT && e < YH + XH) {
+            const int q = e - YH, row = q / (2 * XV), s = q % (2 * XV);
+            const int lx = s < XV ? VX * s : 4 + TX + VX * (s - XV);
+            hgx = x0 - 4 + lx;
+            hgy = y0 + row;
+            c.hl[k] = (row + 4) * LXP + lx;
+        }
+        c.ho[k] = row_off(hgx, hgy, n, (int)sizeof(T));
+        c.hnv[k] = n - hgx;
+    }
+    if (!XT)
+        for (int e = t; e < 2 * 8 * TYL; e += THREADS) {
+            const int b = e / (8 * TYL), q = e % (8 * TYL), row = q >> 3, s = q & 7;
+            tile[b][(row + 4) * LXP + (s < 4 ? s : TX + s)] = T(0);
+        }
+    StRegs<T, HV> R;
+    {
+        V p[4];
 #pragma unroll
-        for (int rr = 0; rr < RPT; rr++) R.q[d][rr] = c.ldv(c.bx, c.co[rr], z0 - 4 + d);
-    sv_side<T, MODE, RPT, W, 0>(R, c, z0);
-    sv_side<T, MODE, RPT, W, 1>(R, c, z0 + 1);
+        for (int q = 0; q < 4; q++) p[q] = c.ld(c.bx, c.co, z0 - 4 + q, c.zlim);
+#pragma unroll
+        for (int q = 0; q < ST_AHEAD; q++) R.F[q] = c.ld(c.bx, c.co, z0 + q, c.zlim);
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+#pragma unroll
+            for (int k = 0; k < HV; k++) R.hq[s][k] = c.ld(c.bx, c.ho[k], z0 + s, z1);
+            if (MODE != ST_LAP) R.vq[s] = c.ld(c.bv, c.co, z0 + s, z1);
+            if (MODE == ST_JAC) R.rq[s] = c.ld(c.br, c.co, z0 + s, z1);
+        }
+#pragma unroll
+        for (int q = 0; q < 3; q++) R.D[q] = p[q + 1] - p[q];  // D_{z0-4+q}
+        R.D[3] = R.F[0] - p[3];
+    }
+    // consecutive planes alternate the two LDS buffers (plane p uses buffer (p - z0) & 1): one barrier per plane then
+    // separates every write of a buffer from the previous reads of it
     int z = z0;
-    for (; z + W <= z1; z += W) {
-        const int b = (z - z0) & 1;
+    for (; z + 8 <= z1; z += 8) {
         auto step = [&](auto sc) {
             constexpr int S = decltype(sc)::value;
-            sv_plane<T, MODE, RPT, W, S, LXP>(R, c, tile, z + S, b ^ (S & 1));
+            st_plane<T, MODE, TXL, TYL, XT, RAG, HV, S>(R, c, tile[S & 1], z + S, z1);
         };
-        PlaneUnroll<0, W>::run(step);
+        PlaneUnroll<0, 8>::run(step);
     }
-    const int b = (z - z0) & 1;
+    // remainder (< 8 planes) with the same slot sequence
     auto tail = [&](auto sc) {
         constexpr int S = decltype(sc)::value;
-        if (z + S < z1) sv_plane<T, MODE, RPT, W, S, LXP>(R, c, tile, z + S, b ^ (S & 1));
+        if (z + S < z1) st_plane<T, MODE, TXL, TYL, XT, RAG, HV, S>(R, c, tile[S & 1], z + S, z1);
     };
-    PlaneUnroll<0, W - 1>::run(tail);
-}
-
-// ---- vector lanes carrying NB bands: lane (tx, ty) owns VX x points of row y0 + ty for bands b0 .. b0 + NB - 1 ----
-// V (and R in ST_JAC per band) is loaded once per point for the NB bands; each band has its own LDS plane.
-template <typename T, int NB, int W> struct VbRegs {
-    typedef typename Vec16<T>::type V;
-    V q[W][NB];
-    V hq[3][NB];
-    V hq2[3][NB];
-    V vq[3];
-    V rq[3][NB];
-};
-
-template <typename T, int NB> struct VbCtx {
-    typedef typename Vec16<T>::type V;
-    static constexpr int VX = Vec16<T>::N;
-    BufRes bx[NB], bo[NB], br[NB], bv;
-    T lamb[NB];
-    unsigned so[NB];   // this lane's store offset per band: co, or BUF_OOB for a band past the block
-    unsigned pb;       // bytes per plane
-    unsigned co;       // centre row (gx, gy): byte offset in a plane, or BUF_OOB
-    unsigned ho, ho2;  // halo vector(s), or BUF_OOB
-    int n;
-    int x0, y0, tx, ty, gx, gy;
-    int h_ly, h_lx;
-    bool has_h, has_h2;
-    T inv_h2, scale, omega, diag_t;
-    __device__ V ldv(BufRes r, unsigned off, int zz) const { return bloadv<T>(r, off + (unsigned)zz * pb); }
-};
-
-template <typename T, int MODE, int NB, int W, int SLOT>
-__device__ __forceinline__ void vb_side(VbRegs<T, NB, W> &R, const VbCtx<T, NB> &c, int zz) {
-    constexpr int QS = SLOT % 3;
-#pragma unroll
-    for (int b = 0; b < NB; b++) {
-        R.hq[QS][b] = c.ldv(c.bx[b], c.ho, zz);
-        if (VbCtx<T, NB>::VX < 4) R.hq2[QS][b] = c.ldv(c.bx[b], c.ho2, zz);
-        if (MODE == ST_JAC) R.rq[QS][b] = c.ldv(c.br[b], c.co, zz);
-    }
-    if (MODE != ST_LAP) R.vq[QS] = c.ldv(c.bv, c.co, zz);
-}
-
-template <typename T, int MODE, int NB, int W, int S, int TYP, int LXP>
-__device__ __forceinline__ void vb_plane(VbRegs<T, NB, W> &R, const VbCtx<T, NB> &c, T (*tile)[NB][TYP][LXP], int z,
-                                         int buf) {
-    typedef typename Vec16<T>::type V;
-    constexpr int VX = Vec16<T>::N;
-    constexpr int C0 = (S + 4) % W;
-    constexpr int NEW = (S + W - 1) % W;
-    constexpr int HS = S % 3;
-#pragma unroll
-    for (int b = 0; b < NB; b++) R.q[NEW][b] = c.ldv(c.bx[b], c.co, z + W - 5);
-    vb_side<T, MODE, NB, W, S + 2>(R, c, z + 2);
-    const int lx = 4 + VX * c.tx, ly = c.ty + 4;
-#pragma unroll
-    for (int b = 0; b < NB; b++) {
-        *reinterpret_cast<V *>(&tile[buf][b][ly][lx]) = R.q[C0][b];
-        if (c.has_h) *reinterpret_cast<V *>(&tile[buf][b][c.h_ly][c.h_lx]) = R.hq[HS][b];
-        if (VX < 4 && c.has_h2) *reinterpret_cast<V *>(&tile[buf][b][c.h_ly][c.h_lx + VX]) = R.hq2[HS][b];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int b = 0; b < NB; b++) {
-        T(*tl)[LXP] = tile[buf][b];
-        T w[VX + 8];
-#pragma unroll
-        for (int q = 0; q < (VX + 8) / VX; q++) {
-            const V vv = *reinterpret_cast<const V *>(&tl[ly][lx - 4 + VX * q]);
-#pragma unroll
-            for (int i = 0; i < VX; i++) w[VX * q + i] = vget<T>(vv, i);
-        }
-        V ym[4], yp[4];
-#pragma unroll
-        for (int m = 1; m <= 4; m++) {
-            ym[m - 1] = *reinterpret_cast<const V *>(&tl[ly - m][lx]);
-            yp[m - 1] = *reinterpret_cast<const V *>(&tl[ly + m][lx]);
-        }
-        V outv;
-#pragma unroll
-        for (int i = 0; i < VX; i++) {
-            const T ce = w[4 + i];
-            const T ax = T(C1) * ((w[5 + i] - ce) + (w[3 + i] - ce)) + T(C2) * ((w[6 + i] - ce) + (w[2 + i] - ce)) +
-                         T(C3) * ((w[7 + i] - ce) + (w[1 + i] - ce)) + T(C4) * ((w[8 + i] - ce) + (w[0 + i] - ce));
-            const T ay = T(C1) * ((vget<T>(yp[0], i) - ce) + (vget<T>(ym[0], i) - ce)) +
-                         T(C2) * ((vget<T>(yp[1], i) - ce) + (vget<T>(ym[1], i) - ce)) +
-                         T(C3) * ((vget<T>(yp[2], i) - ce) + (vget<T>(ym[2], i) - ce)) +
-                         T(C4) * ((vget<T>(yp[3], i) - ce) + (vget<T>(ym[3], i) - ce));
-            const T az = T(C1) * ((vget<T>(R.q[(S + 5) % W][b], i) - ce) + (vget<T>(R.q[(S + 3) % W][b], i) - ce)) +
-                         T(C2) * ((vget<T>(R.q[(S + 6) % W][b], i) - ce) + (vget<T>(R.q[(S + 2) % W][b], i) - ce)) +
-                         T(C3) * ((vget<T>(R.q[(S + 7) % W][b], i) - ce) + (vget<T>(R.q[(S + 1) % W][b], i) - ce)) +
-                         T(C4) * ((vget<T>(R.q[(S + 8) % W][b], i) - ce) + (vget<T>(R.q[S % W][b], i) - ce));
-            const T lap = ((ax + ay) + az) * c.inv_h2;
-            T o;
-            if (MODE == ST_LAP) {
-                o = c.scale * lap;
-            } else if (MODE == ST_HAM) {
-                o = T(-0.5) * lap + vget<T>(R.vq[HS], i) * ce;
-            } else {
-                const T vv = vget<T>(R.vq[HS], i);
-                const T hw = T(-0.5) * lap + vv * ce - c.lamb[b] * ce;
-                T d = c.diag_t + vv - c.lamb[b];
-                d = d > T(0.1) ? d : T(0.1);
-                o = ce + c.omega / d * (vget<T>(R.rq[HS][b], i) - hw);
-            }
-            vset<T>(outv, i, o);
-        }
-        bstorev_nt(outv, c.bo[b], c.so[b] + (unsigned)z * c.pb);
-    }
-}
-
-template <typename T, int MODE, int NB, int W>
-__global__ __launch_bounds__(256) void k_stencil_vb(const T *__restrict__ x, T *__restrict__ out,
-                                                    const T *__restrict__ v, const T *__restrict__ r,
-                                                    const double *__restrict__ lam, int n, long N, int zc, int nb,
-                                                    int order, T inv_h2, T scale, T omega, T diag_t,
-                                                    const T *__restrict__ x2, T *__restrict__ out2, int nb1) {
-    constexpr int VX = Vec16<T>::N;
-    constexpr int TX = 16 * VX, TY = 16;
-    constexpr int LXP = TX + 8, TYP = TY + 8;
-    __shared__ __align__(16) T tile[2][NB][TYP][LXP];
-    VbCtx<T, NB> c;
-    c.tx = threadIdx.x;
-    c.ty = threadIdx.y;
-    const int t = c.ty * 16 + c.tx;
-    const int nzc = (n + zc - 1) / zc;
-    const int ngroups = (nb + NB - 1) / NB;
-    const StWork wk = st_decode((n + TX - 1) / TX, (n + TY - 1) / TY, nzc, ngroups, order);
-    if (!wk.valid) return;
-    c.x0 = wk.tile_x * TX;
-    c.y0 = wk.tile_y * TY;
-    const int z0 = wk.zchunk * zc;
-    const int z1 = min(n, z0 + zc);
-    const long fb = N * (long)sizeof(T);
-    c.n = n;
-    c.pb = (unsigned)((long)n * n * (long)sizeof(T));
-    c.gx = c.x0 + VX * c.tx;
-    c.gy = c.y0 + c.ty;
-    c.co = row_off(c.gx, c.gy, n, (int)sizeof(T));
-#pragma unroll
-    for (int b = 0; b < NB; b++) {
-        const int band = wk.band * NB + b;
-        const bool bok = band < nb;
-        const int bb = bok ? band : wk.band * NB;  // a missing band reads a valid one and stores nothing
-        c.bx[b] = field_res(bb < nb1 ? x + (long)bb * N : x2 + (long)(bb - nb1) * N, fb);
-        c.bo[b] = field_res(bb < nb1 ? out + (long)bb * N : out2 + (long)(bb - nb1) * N, fb);
-        c.br[b] = field_res(MODE == ST_JAC ? r + (long)bb * N : x, MODE == ST_JAC ? fb : 0);
-        c.lamb[b] = MODE == ST_JAC ? (T)lam[bb] : T(0);
-        c.so[b] = bok ? c.co : BUF_OOB;
-    }
-    c.bv = field_res(v, MODE == ST_LAP ? 0 : fb);
-    int h_gx = 0, h_gy = 0;
-    if (t < 128) {
-        const int row = t >> 4, col = t & 15;
-        c.h_ly = row < 4 ? row : TY + row;
-        c.h_lx = 4 + VX * col;
-        h_gx = c.x0 + VX * col;
-        h_gy = c.y0 - 4 + c.h_ly;
-        c.has_h = true;
-    } else if (t < 128 + 2 * TYP) {
-        const int e = t - 128, row = e >> 1, side = e & 1;
-        c.h_ly = row;
-        c.h_lx = side ? 4 + TX : 0;
-        h_gx = side ? c.x0 + TX : c.x0 - 4;
-        h_gy = c.y0 - 4 + row;
-        c.has_h = true;
-    } else {
-        c.h_ly = c.h_lx = 0;
-        c.has_h = false;
-    }
-    c.has_h2 = c.has_h && t >= 128;
-    c.ho = c.has_h ? row_off(h_gx, h_gy, n, (int)sizeof(T)) : BUF_OOB;
-    c.ho2 = c.has_h2 ? row_off(h_gx + VX, h_gy, n, (int)sizeof(T)) : BUF_OOB;
-    c.inv_h2 = inv_h2;
-    c.scale = scale;
-    c.omega = omega;
-    c.diag_t = diag_t;
-    VbRegs<T, NB, W> R;
-#pragma unroll
-    for (int d = 0; d < W - 1; d++)
-#pragma unroll
-        for (int b = 0; b < NB; b++) R.q[d][b] = c.ldv(c.bx[b], c.co, z0 - 4 + d);
-    vb_side<T, MODE, NB, W, 0>(R, c, z0);
-    vb_side<T, MODE, NB, W, 1>(R, c, z0 + 1);
-    int z = z0;
-    for (; z + W <= z1; z += W) {
-        const int b = (z - z0) & 1;
-        auto step = [&](auto sc) {
-            constexpr int S = decltype(sc)::value;
-            vb_plane<T, MODE, NB, W, S, TYP, LXP>(R, c, tile, z + S, b ^ (S & 1));
-        };
-        PlaneUnroll<0, W>::run(step);
-    }
-    const int b = (z - z0) & 1;
-    auto tail = [&](auto sc) {
-        constexpr int S = decltype(sc)::value;
-        if (z + S < z1) vb_plane<T, MODE, NB, W, S, TYP, LXP>(R, c, tile, z + S, b ^ (S & 1));
-    };
-    PlaneUnroll<0, W - 1>::run(tail);
+    PlaneUnroll<0, 7>::run(tail);
 }
 
 struct StVariant {
-    int rpt;
-    int zc;     // 0 = whole column
-    int vec;    // 1: 16-byte vector lanes (needs n divisible by the vector width); 2: lanes carrying rpt bands;
-                // 3: scalar lanes on a 32-wide tile (rpt 1 or 2)
+    int tx;     // tile width in points
+    int zc;     // planes per chunk; 0: whole columns, -1: chunks that load the CUs evenly
     int order;  // XCD work order: 0 tiles fastest, 1 bands fastest, G >= 2 bands in groups of G fastest
-    int win;    // z window: 9 (no look-ahead beyond the taps) or 12 (three planes of look-ahead)
     const char *name;
 };
 static const StVariant ST_VARIANTS[] = {
-    {4, 0, 0, 0, 9, "64x16 tile, full z column"},
-    {4, 32, 0, 0, 9, "64x16 tile, z chunks of 32"},
-    {4, 16, 0, 0, 9, "64x16 tile, z chunks of 16"},
-    {2, 0, 0, 0, 9, "64x8 tile, full z column"},
-    {2, 16, 0, 0, 9, "64x8 tile, z chunks of 16"},
-    {2, 8, 0, 0, 9, "64x8 tile, z chunks of 8"},
-    {1, 0, 1, 0, 9, "vector lanes, 16 rows, full z column"},
-    {1, 32, 1, 0, 9, "vector lanes, 16 rows, z chunks of 32"},
-    {1, 16, 1, 0, 9, "vector lanes, 16 rows, z chunks of 16"},
-    {2, 0, 1, 0, 9, "vector lanes, 32 rows, full z column"},
-    {2, 32, 1, 0, 9, "vector lanes, 32 rows, z chunks of 32"},
-    {1, 0, 1, 1, 9, "vector lanes, 16 rows, full z column, bands fastest"},
-    {1, 32, 1, 1, 9, "vector lanes, 16 rows, z chunks of 32, bands fastest"},
-    {2, 0, 1, 1, 9, "vector lanes, 32 rows, full z column, bands fastest"},
-    {2, 0, 0, 1, 9, "64x8 tile, full z column, bands fastest"},
-    {2, 16, 0, 1, 9, "64x8 tile, z chunks of 16, bands fastest"},
-    {2, 0, 2, 0, 9, "vector lanes, 2 bands per lane, full z column"},
-    {2, 32, 2, 0, 9, "vector lanes, 2 bands per lane, z chunks of 32"},
-    {2, 0, 2, 1, 9, "vector lanes, 2 bands per lane, full z column, bands fastest"},
-    {4, 0, 2, 0, 9, "vector lanes, 4 bands per lane, full z column"},
-    {1, 0, 1, 8, 9, "vector lanes, 16 rows, full z column, bands in groups of 8"},
-    {1, 0, 1, 4, 9, "vector lanes, 16 rows, full z column, bands in groups of 4"},
-    {2, 0, 1, 8, 9, "vector lanes, 32 rows, full z column, bands in groups of 8"},
-    {1, 32, 1, 8, 9, "vector lanes, 16 rows, z chunks of 32, bands in groups of 8"},
-    {4, 0, 0, 8, 9, "64x16 tile, full z column, bands in groups of 8"},
-    {2, 16, 0, 8, 9, "64x8 tile, z chunks of 16, bands in groups of 8"},
-    {2, 16, 0, 4, 9, "64x8 tile, z chunks of 16, bands in groups of 4"},
-    {4, 0, 0, 0, 12, "64x16 tile, full z column, 12-plane window"},
-    {4, 32, 0, 0, 12, "64x16 tile, z chunks of 32, 12-plane window"},
-    {2, 0, 0, 0, 12, "64x8 tile, full z column, 12-plane window"},
-    {2, 16, 0, 0, 12, "64x8 tile, z chunks of 16, 12-plane window"},
-    {2, 16, 0, 4, 12, "64x8 tile, z chunks of 16, bands in groups of 4, 12-plane window"},
-    {1, 0, 1, 0, 12, "vector lanes, 16 rows, full z column, 12-plane window"},
-    {1, 32, 1, 0, 12, "vector lanes, 16 rows, z chunks of 32, 12-plane window"},
-    {1, 0, 1, 4, 12, "vector lanes, 16 rows, full z column, bands in groups of 4, 12-plane window"},
-    {2, 0, 1, 0, 12, "vector lanes, 32 rows, full z column, 12-plane window"},
-    {2, 0, 2, 0, 12, "vector lanes, 2 bands per lane, full z column, 12-plane window"},
-    {2, 0, 3, 0, 9, "32x16 tile, full z column"},
-    {2, 16, 3, 0, 9, "32x16 tile, z chunks of 16"},
-    {1, 0, 3, 0, 9, "32x8 tile, full z column"},
-    {1, 16, 3, 0, 9, "32x8 tile, z chunks of 16"},
-    {2, 16, 3, 1, 9, "32x16 tile, z chunks of 16, bands fastest"},
-    {2, 16, 3, 4, 9, "32x16 tile, z chunks of 16, bands in groups of 4"},
+    {32, -1, 0, "32-wide tile, balanced z chunks"},
+    {32, 0, 0, "32-wide tile, full z column"},
+    {32, 32, 0, "32-wide tile, z chunks of 32"},
+    {32, 16, 0, "32-wide tile, z chunks of 16"},
+    {32, 8, 0, "32-wide tile, z chunks of 8"},
+    {64, -1, 0, "64-wide tile, balanced z chunks"},
+    {64, 0, 0, "64-wide tile, full z column"},
+    {64, 32, 0, "64-wide tile, z chunks of 32"},
+    {64, 16, 0, "64-wide tile, z chunks of 16"},
+    {64, 8, 0, "64-wide tile, z chunks of 8"},
+    {64, 0, 4, "64-wide tile, full z column, bands in groups of 4"},
+    {64, 24, 4, "64-wide tile, z chunks of 24, bands in groups of 4"},
+    {96, -1, 0, "96-wide tile, balanced z chunks"},
+    {96, 0, 0, "96-wide tile, full z column"},
+    {96, 32, 0, "96-wide tile, z chunks of 32"},
+    {96, 16, 0, "96-wide tile, z chunks of 16"},
+    {96, 8, 0, "96-wide tile, z chunks of 8"},
+    {128, -1, 0, "128-wide tile, balanced z chunks"},
+    {128, 0, 0, "128-wide tile, full z column"},
+    {128, 32, 0, "128-wide tile, z chunks of 32"},
+    {128, 16, 0, "128-wide tile, z chunks of 16"},
+    {128, 8, 0, "128-wide tile, z chunks of 8"},
+    {192, -1, 0, "192-wide tile, balanced z chunks"},
+    {192, 0, 0, "192-wide tile, full z column"},
+    {192, 32, 0, "192-wide tile, z chunks of 32"},
+    {192, 16, 0, "192-wide tile, z chunks of 16"},
+    {192, 8, 0, "192-wide tile, z chunks of 8"},
+    {192, 0, 4, "192-wide tile, full z column, bands in groups of 4"},
+    {192, 24, 4, "192-wide tile, z chunks of 24, bands in groups of 4"},
 };
 static int g_default_variant[2] = {-1, -1};
 
@@ -805,129 +471,92 @@ int stencil_variants() { return (int)(sizeof(ST_VARIANTS) / sizeof(ST_VARIANTS[0
 const char *stencil_variant_name(int v) { return (v >= 0 && v < stencil_variants()) ? ST_VARIANTS[v].name : "auto"; }
 void stencil_set_default_variant(int dtype_size, int variant) { g_default_variant[dtype_size == 8 ? 1 : 0] = variant; }
 
-// Heuristic when no tuned choice exists: whole columns when the band x tile count alone fills the chip, z chunks
-// otherwise (small grids, few bands).
-static int pick_variant(int n, int nb) {
-    long tiles16 = (long)((n + 63) / 64) * ((n + 15) / 16) * nb;
-    if (tiles16 >= 1024) return 0;
-    if (tiles16 * ((n + 31) / 32) >= 1024) return 1;
-    return 2;
+// rows and waves of the tile of each width (the TXL x TYL of stencil_dispatch)
+static int st_rows(int tx, int esize) { return esize == 4 ? (tx == 32 ? 32 : tx == 192 ? 8 : 16) : (tx <= 64 ? 16 : 8); }
+static int st_waves(int tx, int esize) { return tx / (16 / esize) * st_rows(tx, esize) / 64; }
+
+// The balanced chunk: a chunk of zc planes streams zc + 8, and the launch takes as long as its fullest CU. With w waves
+// on a CU a plane step took about max(7, w) in one unit (0.09 us) wherever it was measured (95^3 f32, 96-wide tiles: 7
+// bands, 252 blocks of 6 waves in chunks of 16, 13.9 us; 504 blocks in chunks of 8, 16.8 us; 336 in chunks of 12,
+// > 17.4 us; 16 bands, 480 blocks in chunks of 19, 31.2 us; 576 in chunks of 16, 37.1 us). f32 tiles on rows that do not
+// fit one tile keep chunks of at most 16 planes, whose tiles meet in the L2s (160^3 x 46 sweep: 477 us, 490 in chunks of
+// 32).
+static int st_chunk(int tx, int n, int nb, int esize) {
+    const int rows = st_rows(tx, esize), waves = st_waves(tx, esize);
+    const long cols = (long)((n + tx - 1) / tx) * ((n + rows - 1) / rows) * nb;
+    int best = n, zc = esize == 4 && n > 128 && tx < n ? std::min(n, 16) : n;
+    double best_cost = 1e300;
+    do {
+        const int nzc = (n + zc - 1) / zc;
+        zc = (n + nzc - 1) / nzc;
+        const double per_cu = (double)((cols * nzc + 255) / 256);
+        const double cost = (zc + 8) * std::max(7.0, per_cu * waves);
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = zc;
+        }
+        zc--;
+    } while (zc >= 2);
+    return best;
 }
 
-template <typename T, int MODE, int RPT, int W, int TX>
+// The tile when no tuned choice exists: the narrowest one that takes whole rows up to 128 points (no x halos), in f32
+// also 192-wide rows that fill it; 64-wide otherwise; in balanced chunks. Over 66 shapes (25^3 .. 256^3, 1 .. 32 bands,
+// three modes, both types) its time was within 3 % of the best variant's in the geometric mean.
+static int pick_variant(int n, int esize) {
+    const int tx = n <= 64 ? 64 : n <= 96 ? 96 : n <= 128 ? 128 : esize == 4 && n > 176 && n <= 192 ? 192 : 64;
+    for (int v = 0; v < stencil_variants(); v++)
+        if (ST_VARIANTS[v].tx == tx && ST_VARIANTS[v].zc == -1) return v;
+    return 0;
+}
+
+template <typename T, int MODE, int TXL, int TYL, bool XT>
 static void launch_stencil(const StencilParams &p, int zc, int order, const T *x, T *out, const T *v, const T *r,
                            const double *lam, hipStream_t s) {
-    constexpr int TYB = 256 / TX, TY = TYB * RPT;
+    constexpr int VX = Vec16<T>::N, TX = TXL * VX;
     const int n = p.n;
     const long N = (long)n * n * n;
-    if (zc <= 0 || zc > n) zc = n;
+    if (zc < 0) zc = st_chunk(TX, n, p.nb, (int)sizeof(T));
+    if (zc == 0 || zc > n) zc = n;
     const int nzc = (n + zc - 1) / zc;
-    const unsigned grid = st_grid((n + TX - 1) / TX, (n + TY - 1) / TY, nzc, p.nb, order);
-    dim3 block(TX, TYB, 1);
-    hipLaunchKernelGGL((k_stencil<T, MODE, RPT, W, TX>), dim3(grid), block, 0, s, x, out, v, r, lam, n, N, zc, p.nb, order,
-                       (T)(1.0 / (p.h * p.h)), (T)p.scale, (T)p.omega, (T)p.diag_t, static_cast<const T *>(p.x2),
-                       static_cast<T *>(p.out2), p.nb1 < 0 ? p.nb : p.nb1);
+    const dim3 grid(st_grid((n + TX - 1) / TX, (n + TYL - 1) / TYL, nzc, p.nb, order)), block(TXL * TYL);
+    const double inv_h2 = 1.0 / (p.h * p.h);
+    const T hs = (T)(MODE == ST_LAP ? p.scale * inv_h2 : -0.5 * inv_h2);
+    const int nb1 = p.nb1 < 0 ? p.nb : p.nb1;
+#define LIRA_GO(RAG_)                                                                                                   \
+    hipLaunchKernelGGL((k_stencil<T, MODE, TXL, TYL, XT, RAG_>), grid, block, 0, s, x, out, v, r, lam, n, N, zc, p.nb, \
+                       order, hs, (T)p.omega, (T)p.diag_t, static_cast<const T *>(p.x2), static_cast<T *>(p.out2), nb1)
+    if (n % VX) LIRA_GO(true);
+    else LIRA_GO(false);
+#undef LIRA_GO
     LIRA_HIP(hipGetLastError());
 }
 
-template <typename T, int MODE, int RPT, int W>
-static void launch_stencil_vec(const StencilParams &p, int zc, int order, const T *x, T *out, const T *v, const T *r,
-                               const double *lam, hipStream_t s) {
-    constexpr int VX = Vec16<T>::N;
-    const int n = p.n;
-    const long N = (long)n * n * n;
-    if (zc <= 0 || zc > n) zc = n;
-    const int nzc = (n + zc - 1) / zc;
-    const unsigned grid = st_grid((n + 16 * VX - 1) / (16 * VX), (n + 16 * RPT - 1) / (16 * RPT), nzc, p.nb, order);
-    hipLaunchKernelGGL((k_stencil_vec<T, MODE, RPT, W>), dim3(grid), dim3(16, 16, 1), 0, s, x, out, v, r, lam, n, N, zc,
-                       p.nb, order, (T)(1.0 / (p.h * p.h)), (T)p.scale, (T)p.omega, (T)p.diag_t,
-                       static_cast<const T *>(p.x2), static_cast<T *>(p.out2), p.nb1 < 0 ? p.nb : p.nb1);
-    LIRA_HIP(hipGetLastError());
-}
-
-template <typename T, int MODE, int NB, int W>
-static void launch_stencil_vb(const StencilParams &p, int zc, int order, const T *x, T *out, const T *v, const T *r,
-                              const double *lam, hipStream_t s) {
-    constexpr int VX = Vec16<T>::N;
-    const int n = p.n;
-    const long N = (long)n * n * n;
-    if (zc <= 0 || zc > n) zc = n;
-    const int nzc = (n + zc - 1) / zc;
-    const unsigned grid = st_grid((n + 16 * VX - 1) / (16 * VX), (n + 15) / 16, nzc, (p.nb + NB - 1) / NB, order);
-    hipLaunchKernelGGL((k_stencil_vb<T, MODE, NB, W>), dim3(grid), dim3(16, 16, 1), 0, s, x, out, v, r, lam, n, N, zc,
-                       p.nb, order, (T)(1.0 / (p.h * p.h)), (T)p.scale, (T)p.omega, (T)p.diag_t,
-                       static_cast<const T *>(p.x2), static_cast<T *>(p.out2), p.nb1 < 0 ? p.nb : p.nb1);
-    LIRA_HIP(hipGetLastError());
-}
-
-// launch the variant's kernel for window W (4 bands per lane exist only at W = 9: their registers)
-template <typename T, int W>
-static void stencil_dispatch(int mode, const StVariant &sv, const StencilParams &p, const T *x, T *out, const T *v,
-                             const T *r, const double *lam, hipStream_t s) {
-#define LIRA_VB(MODE_, NB_) launch_stencil_vb<T, MODE_, NB_, W>(p, sv.zc, sv.order, x, out, v, r, lam, s)
-#define LIRA_SV(MODE_, RPT_) launch_stencil_vec<T, MODE_, RPT_, W>(p, sv.zc, sv.order, x, out, v, r, lam, s)
-#define LIRA_ST(MODE_, RPT_) launch_stencil<T, MODE_, RPT_, W, 64>(p, sv.zc, sv.order, x, out, v, r, lam, s)
-#define LIRA_ST32(MODE_, RPT_) launch_stencil<T, MODE_, RPT_, W, 32>(p, sv.zc, sv.order, x, out, v, r, lam, s)
-    if (sv.vec == 2) {
-        bool four = false;
-        if constexpr (W == 9) {
-            if (sv.rpt == 4) {
-                four = true;
-                if (mode == ST_LAP) LIRA_VB(ST_LAP, 4);
-                else if (mode == ST_HAM) LIRA_VB(ST_HAM, 4);
-                else LIRA_VB(ST_JAC, 4);
-            }
-        }
-        if (!four) {
-            if (mode == ST_LAP) LIRA_VB(ST_LAP, 2);
-            else if (mode == ST_HAM) LIRA_VB(ST_HAM, 2);
-            else LIRA_VB(ST_JAC, 2);
-        }
-    } else if (sv.vec == 1) {
-        if (sv.rpt == 1) {
-            if (mode == ST_LAP) LIRA_SV(ST_LAP, 1);
-            else if (mode == ST_HAM) LIRA_SV(ST_HAM, 1);
-            else LIRA_SV(ST_JAC, 1);
-        } else {
-            if (mode == ST_LAP) LIRA_SV(ST_LAP, 2);
-            else if (mode == ST_HAM) LIRA_SV(ST_HAM, 2);
-            else LIRA_SV(ST_JAC, 2);
-        }
-    } else if (sv.vec == 3) {
-        bool done = false;
-        if constexpr (W == 9) {
-            done = true;
-            if (sv.rpt == 1) {
-                if (mode == ST_LAP) LIRA_ST32(ST_LAP, 1);
-                else if (mode == ST_HAM) LIRA_ST32(ST_HAM, 1);
-                else LIRA_ST32(ST_JAC, 1);
-            } else {
-                if (mode == ST_LAP) LIRA_ST32(ST_LAP, 2);
-                else if (mode == ST_HAM) LIRA_ST32(ST_HAM, 2);
-                else LIRA_ST32(ST_JAC, 2);
-            }
-        }
-        if (!done) throw InvalidError("stencil: 32-wide tiles exist only with the 9-plane window");
-    } else if (sv.rpt == 4) {
-        if (mode == ST_LAP) LIRA_ST(ST_LAP, 4);
-        else if (mode == ST_HAM) LIRA_ST(ST_HAM, 4);
-        else LIRA_ST(ST_JAC, 4);
+// the tile of each width: TXL lanes x TYL rows
+template <typename T, int MODE>
+static void stencil_dispatch(const StVariant &sv, const StencilParams &p, const T *x, T *out, const T *v, const T *r,
+                             const double *lam, hipStream_t s) {
+#define LIRA_ST(TXL_, TYL_, XT_) launch_stencil<T, MODE, TXL_, TYL_, XT_>(p, sv.zc, sv.order, x, out, v, r, lam, s)
+    if constexpr (sizeof(T) == 4) {
+        if (sv.tx == 32) LIRA_ST(8, 32, true);
+        else if (sv.tx == 64) LIRA_ST(16, 16, true);
+        else if (sv.tx == 96) LIRA_ST(24, 16, false);
+        else if (sv.tx == 128) LIRA_ST(32, 16, false);
+        else LIRA_ST(48, 8, false);
     } else {
-        if (mode == ST_LAP) LIRA_ST(ST_LAP, 2);
-        else if (mode == ST_HAM) LIRA_ST(ST_HAM, 2);
-        else LIRA_ST(ST_JAC, 2);
+        if (sv.tx == 32) LIRA_ST(16, 16, true);
+        else if (sv.tx == 64) LIRA_ST(32, 16, true);
+        else if (sv.tx == 96) LIRA_ST(48, 8, false);
+        else LIRA_ST(64, 8, false);
     }
-#undef LIRA_VB
-#undef LIRA_SV
 #undef LIRA_ST
-#undef LIRA_ST32
 }
 
+// a tile of 96 or more columns takes the whole row
 bool stencil_variant_usable(int variant, int n, int dtype_size) {
     if (variant < 0 || variant >= stencil_variants()) return false;
-    const int vec = ST_VARIANTS[variant].vec;
-    if (vec == 0 || vec == 3) return true;
-    return n % (16 / dtype_size) == 0;
+    const int tx = ST_VARIANTS[variant].tx;
+    return tx <= 64 || (n <= tx && (tx < 192 || dtype_size == 4));
 }
 
 template <typename T>
@@ -943,17 +572,11 @@ void stencil(int mode, const StencilParams &p, const T *x, T *out, const T *v, c
         throw InvalidError("stencil: grid too large for 32-bit field offsets ((n^3 + 4 n^2) values must stay below "
                            "2^31 bytes)");
     if (variant < 0) variant = g_default_variant[sizeof(T) == 8 ? 1 : 0];
-    if (!stencil_variant_usable(variant, p.n, (int)sizeof(T))) variant = pick_variant(p.n, p.nb);
-    if (ST_VARIANTS[variant].vec == 1 || ST_VARIANTS[variant].vec == 2) {
-        // vector lanes need 16-byte aligned bases (every band then stays aligned since n is a multiple of the width)
-        auto misaligned = [](const void *q) { return q && (reinterpret_cast<uintptr_t>(q) & 15) != 0; };
-        if (misaligned(x) || misaligned(out) || misaligned(v) || misaligned(r) || misaligned(p.x2) ||
-            misaligned(p.out2))
-            variant = pick_variant(p.n, p.nb);
-    }
+    if (!stencil_variant_usable(variant, p.n, (int)sizeof(T))) variant = pick_variant(p.n, (int)sizeof(T));
     const StVariant &sv = ST_VARIANTS[variant];
-    if (sv.win == 12) stencil_dispatch<T, 12>(mode, sv, p, x, out, v, r, lam, s);
-    else stencil_dispatch<T, 9>(mode, sv, p, x, out, v, r, lam, s);
+    if (mode == ST_LAP) stencil_dispatch<T, ST_LAP>(sv, p, x, out, v, r, lam, s);
+    else if (mode == ST_HAM) stencil_dispatch<T, ST_HAM>(sv, p, x, out, v, r, lam, s);
+    else stencil_dispatch<T, ST_JAC>(sv, p, x, out, v, r, lam, s);
 }
 
 
