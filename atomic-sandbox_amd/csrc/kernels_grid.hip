@@ -1,6 +1,7 @@
 // gfx950 kernels on the dense n^3 grid: the block stencil H.X, reductions, the tall-skinny Gram S^T U, block
 // linear combinations, density accumulation, LSDA, nuclear potential, orbital guess, DIIS mix and HF forces.
 // All kernels are written for 64-wide wavefronts; reductions are deterministic (fixed partial counts, fixed order).
+#include "lira.h"
 #include "lira_internal.hpp"
 #include "lsda.hpp"
 
@@ -668,9 +669,6 @@ void reduce_jobs(const RedJobs<T> &jobs, int n, double scale, double *partials, 
 }
 
 // ------------------------------------------------------------------------------------------- Gram ----
-// G = scale S^T U over N points. A workgroup computes a 32 (S) x 64 (U) output block over one chunk of points,
-// staging 64 points of its 96 columns in LDS at a time; each thread owns a 2 x 4 register tile accumulated in f64.
-
 // A load through a pointer the compiler cannot place (one read from an LDS table of column bases) becomes a flat
 // load, which also counts against the LDS wait counter: every wait for an LDS read would then wait for the loads in
 // flight as well. Column data is always global memory, so these loads name that address space.
@@ -700,49 +698,26 @@ __device__ inline const void *col_base(const ColPtrs &c, int col, long N, int es
     return static_cast<const char *>(c.base[s]) + (size_t)(col - c.start[s]) * (size_t)N * (size_t)esize;
 }
 
-// G = scale S^T U on the f64 matrix cores: v_mfma_f64_16x16x4f64 with A = S-columns x 4 points, B = 4 points x
-// U-columns (lane l holds A[l % 16][l / 16] and B[l / 16][l % 16]; the 16 x 16 result lands as D[l / 16 + 4 r][l % 16]
-// in register r, measured on gfx950). A workgroup (4 waves) owns a 32 x 64 output tile over one chunk of points; each wave two 16 x 16
-// sub-tiles. Columns are staged 32 points at a time in LDS as f64 (f32 inputs convert exactly), so the products are
-// exact and the accumulation is f64 in every precision mode.
+// G = scale S^T U on the f64 matrix cores: v_mfma_f64_16x16x4f64 with A = 16 S columns x 4 points, B = 4 points x 16 U
+// columns (lane l holds A[l % 16][l / 16] and B[l / 16][l % 16]; the 16 x 16 result lands as D[l / 16 + 4 r][l % 16] in
+// register r, measured on gfx950). Inputs convert to f64 exactly, so the products are exact and the accumulation is f64
+// in every precision mode.
+//
+// The operands go from memory to the matrix cores without LDS. The order in which points enter the sum is free, so a lane
+// loads four consecutive points of its column (16 bytes in f32, 32 in f64: column l % 16 of a 16-column block, points
+// 4 (l / 16) .. + 3 of a 16-point stage) and feeds one of them to each of four MFMAs; A and B share that layout, so a
+// column block that is both (S^T S, SHARE) is loaded once. A wave holds RB x CB output blocks: per 16 points RB + CB
+// loads and conversions of 4 values against 4 RB CB MFMAs (64 cycles each), one unit of 16 H points in flight while the
+// previous one is multiplied. The waves of a workgroup take interleaved units of its chunk of points and their blocks
+// are summed in wave order; the workgroups that share a chunk run next to each other on one XCD, so its columns
+// come from that L2. (Before, each wave staged its columns through LDS as f64 with a pointer lookup per load: 24 x 48
+// columns on 95^3 f32 60 us, 138 x 276 on 160^3 11 ms.)
 typedef double lira_d4 __attribute__((ext_vector_type(4)));
-constexpr int G2_TI = 32, G2_TJ = 64;
 
-// Each wave streams its own 16-point stages through a private LDS slice (96 columns x 16 points): no block barrier
-// in the loop, so the four waves of a workgroup never wait on each other. A stage is 24 elements per lane
-// (consecutive lanes on consecutive points of one column: 16 lanes read 16 contiguous values), loaded into registers
-// one stage ahead so their latency hides behind the 32 MFMAs of the current stage. The four waves take interleaved
-// stages of the workgroup's chunk; their 32 x 64 accumulators are summed in a fixed order at the end.
-constexpr int G2_S = 16;  // points per wave stage
-// A wave's slab slice holds the 4 LOADS rows a stage loads (the tile's 32 S rows, then the packed U rows) and, last,
-// a row that stays zero (the B operand of a U column past q): sized by LOADS, the slab of the common 16-load shape
-// takes 35 KB instead of the 53 KB of the widest, and four workgroups fit a CU's LDS instead of two.
-template <int LOADS> constexpr int g2_rows() { return 4 * LOADS + 1; }
-
-// Every load is issued unconditionally and its value is not touched until the stage is staged: a missing column or a
-// point past the chunk reads a zero constant instead. (A load under a branch, or a select on the loaded value, makes
-// the compiler wait for the load at once, and the stage-ahead prefetch would never be in flight.)
-template <typename T> struct GramZero;
-template <> struct GramZero<float> { static __device__ const float *ptr(); };
-template <> struct GramZero<double> { static __device__ const double *ptr(); };
-__device__ const float lira_gram_zero_f = 0.0f;
-__device__ const double lira_gram_zero_d = 0.0;
-__device__ const float *GramZero<float>::ptr() { return &lira_gram_zero_f; }
-__device__ const double *GramZero<double>::ptr() { return &lira_gram_zero_d; }
-
-template <typename T, int LOADS>
-__device__ inline void gram_fetch(const T *const *cols, long p0, long p_end, T (&v)[LOADS]) {
-    const int lane = threadIdx.x & 63;
-    const T *zero = GramZero<T>::ptr();
-#pragma unroll
-    for (int u = 0; u < LOADS; u++) {
-        const int e = lane + 64 * u;
-        const int col = e >> 4, pp = e & 15;
-        const long p = p0 + pp;
-        const T *c = cols[col];
-        v[u] = gload(c != nullptr && p < p_end ? c + p : zero);
-    }
-}
+// four consecutive values at any element alignment, in the global address space
+template <typename T> struct Quad {
+    typedef T type __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+};
 
 // With sym (U's first m columns are S's), the 16 x 16 blocks of S^T S strictly below its diagonal are skipped
 // (gram_mirrored): k_gram_finish reads their values from the transposed block, the same sum of the same exact products.
@@ -751,145 +726,136 @@ __host__ __device__ inline bool gram_mirrored(int sym, int m, int i, int j) {
     return sym && cb < rb && 16 * (cb + 1) <= m;
 }
 
-// The slab holds the tile's 32 S columns in rows 0..31 and, packed after them, only the U columns that are neither past
-// q nor one of the tile's S columns (U = [S, R, HW, HP] in LOBPCG): each U column reads its B operand from its packed
-// row, its S row, or the zero row. LOADS = 8 (the S rows) + a quarter of the packed U columns, rounded up to a
-// multiple of 4: the elements each lane loads per 16-point stage.
-// At least three waves per SIMD: the compiler then keeps the accumulators in VGPRs (128 registers at 16 loads, four
-// waves) instead of 138 VGPRs + 64 AGPRs (two waves), with no spills; the loads of more waves are in flight at once.
-template <typename T, int LOADS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_gram(ColPtrs S, ColPtrs U, int m,
-                                                                                     int q, long N, long chunk,
-                                              double *partials, int sym) {
-    constexpr int ROWS = g2_rows<LOADS>(), ZERO_ROW = ROWS - 1;
-    static_assert(4 * ROWS * (G2_S + 1) >= 3 * 16 * 64, "the final reduction's half pass must fit the slab");
-    __shared__ double slab[4][ROWS][G2_S + 1];  // one slice per wave; reused for the final reduction
-    __shared__ const T *cols[G2_TI + G2_TJ];
-    __shared__ int urow[G2_TJ];  // the slab row each U column's B operand is read from
-    const int nbj = (q + G2_TJ - 1) / G2_TJ;
-    const int bi = blockIdx.y / nbj, bj = blockIdx.y - bi * nbj;
-    const int i0 = bi * G2_TI, j0 = bj * G2_TJ;
-    const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-    // which 16 x 16 output blocks this tile computes (uniform over the workgroup); a tile with none returns here,
-    // before any barrier
-    const int ni = min(2, (m - i0 + 15) / 16), nj = min(4, (q - j0 + 15) / 16);
-    bool live[2][4];
-    bool any = false;
+// W waves of a workgroup
+__host__ __device__ constexpr int gram_waves(int RB, int CB, bool SHARE) {
+    return !SHARE ? 4 : RB * CB <= 6 && CB <= 3 ? 16 : 8;
+}
+template <typename T, int RB, int CB, bool SHARE, int H>
+__global__ __launch_bounds__(64 * gram_waves(RB, CB, SHARE), gram_waves(RB, CB, SHARE) == 16 ? 4 : 2) void k_gram(ColPtrs S, ColPtrs U, int m, int q, long N, long chunk, int chunks, int nc,
+                                              int nsub, double *partials, int sym) {
+    typedef typename Quad<T>::type Q;
+    constexpr int UP = 16 * H;           // points of a wave's unit
+    constexpr int NB = SHARE ? CB : RB + CB;  // column blocks loaded
+    constexpr int W = gram_waves(RB, CB, SHARE);
+    __shared__ double red[W][256];
+    const int total = chunks * nsub, per = (total + 7) / 8;
+    const int L = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || L >= total) return;
+    const int ch = L / nsub, sub = L - ch * nsub, bi = sub / nc, bj = sub - bi * nc;
+    const int i0 = bi * RB * 16, j0 = bj * CB * 16;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int c16 = lane & 15, k4 = lane >> 4;
+    // the output blocks this tile computes; a tile with none returns here, before any barrier
+    unsigned live = 0;
 #pragma unroll
-    for (int a = 0; a < 2; a++)
+    for (int a = 0; a < RB; a++)
 #pragma unroll
-        for (int b = 0; b < 4; b++) {
-            live[a][b] = a < ni && b < nj && !gram_mirrored(sym, m, i0 + 16 * a, j0 + 16 * b);
-            any = any || live[a][b];
-        }
-    if (!any) return;
-    if (t < G2_TI) cols[t] = i0 + t < m ? static_cast<const T *>(col_base(S, i0 + t, N, sizeof(T))) : nullptr;
-    if (t >= 64 + G2_TI && t < 64 + G2_TI + G2_TJ) cols[t - 64] = nullptr;  // packed U rows default to zero loads
-    __syncthreads();
-    if (wave == 1) {
-        // U column c = lane: an alias of one of the tile's S columns, a real column (packed in ballot order), or none
-        const int c = lane;
-        const T *uc = j0 + c < q ? static_cast<const T *>(col_base(U, j0 + c, N, sizeof(T))) : nullptr;
-        int srow = -1;
-        if (uc)
-            for (int i = 0; i < G2_TI; i++)
-                if (cols[i] == uc) {
-                    srow = i;
-                    break;
-                }
-        const bool real = uc != nullptr && srow < 0;
-        const unsigned long long mask = __ballot(real);
-        const int rank = __popcll(mask & ((1ull << c) - 1ull));
-        urow[c] = srow >= 0 ? srow : real ? G2_TI + rank : ZERO_ROW;
-        if (real) cols[G2_TI + rank] = uc;
+        for (int b = 0; b < CB; b++)
+            if (i0 + 16 * a < m && j0 + 16 * b < q && !gram_mirrored(sym, m, i0 + 16 * a, j0 + 16 * b))
+                live |= 1u << (a * CB + b);
+    if (live == 0) return;
+    // this lane's column of each block; past the last column it reads that one (its outputs are not stored)
+    const T *col[NB];
+#pragma unroll
+    for (int b = 0; b < CB; b++) col[b] = static_cast<const T *>(col_base(U, min(j0 + 16 * b + c16, q - 1), N, sizeof(T)));
+    if constexpr (!SHARE) {
+#pragma unroll
+        for (int a = 0; a < RB; a++)
+            col[CB + a] = static_cast<const T *>(col_base(S, min(i0 + 16 * a + c16, m - 1), N, sizeof(T)));
     }
-    // the zero row of every wave's slice
-    if (lane < G2_S) slab[wave][ZERO_ROW][lane] = 0.0;
-    lira_d4 acc[2][4];
+    lira_d4 acc[RB][CB];
 #pragma unroll
-    for (int a = 0; a < 2; a++)
+    for (int a = 0; a < RB; a++)
 #pragma unroll
-        for (int b = 0; b < 4; b++) acc[a][b] = lira_d4{0.0, 0.0, 0.0, 0.0};
-    const long p_begin = (long)blockIdx.x * chunk;
-    const long p_end = min(N, p_begin + chunk);
-    __syncthreads();
-    double(*sl)[G2_S + 1] = slab[wave];
-    // two stage buffers in registers: the loads of the stage after next are in flight while a stage is consumed
-    T va[LOADS], vb[LOADS];
-    long p0 = p_begin + (long)wave * G2_S;
-    gram_fetch<T, LOADS>(cols, p0, p_end, va);
-    gram_fetch<T, LOADS>(cols, p0 + 4 * G2_S, p_end, vb);
-    const int r16 = lane & 15, k4 = lane >> 4;
-    int brow[4];
+        for (int b = 0; b < CB; b++) acc[a][b] = lira_d4{0.0, 0.0, 0.0, 0.0};
+    const long p_begin = (long)ch * chunk, p_end = min(N, p_begin + chunk);
+    const long units = p_end > p_begin ? (p_end - p_begin) / UP : 0;  // whole units; the rest is the last chunk's tail
+    // the products of one unit; ALL: every block of the tile is live. (A SHARE tile is the whole product, so its dead
+    // blocks are those with b < a, known here.)
+    auto multiply = [&](const Q(&v)[H][NB], auto all) {
 #pragma unroll
-    for (int b = 0; b < 4; b++) brow[b] = urow[16 * b + r16];
-    // one stage: stage v into the wave's slice, refill v with the stage two ahead (past the chunk: zeros), then the
-    // MFMAs of the staged points
-    auto stage = [&](T(&v)[LOADS], long pn) {
+        for (int h = 0; h < H; h++)
 #pragma unroll
-        for (int u = 0; u < LOADS; u++) {
-            const int e = lane + 64 * u;
-            sl[e >> 4][e & 15] = (double)v[u];
+            for (int j = 0; j < 4; j++) {
+                double x[NB];
+#pragma unroll
+                for (int b = 0; b < NB; b++) x[b] = (double)v[h][b][j];
+#pragma unroll
+                for (int a = 0; a < RB; a++)
+#pragma unroll
+                    for (int b = SHARE ? a : 0; b < CB; b++)
+                        if (SHARE || decltype(all)::value || (live >> (a * CB + b)) & 1u)
+                            acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[SHARE ? a : CB + a], x[b], acc[a][b], 0, 0, 0);
+            }
+    };
+    auto run = [&](auto all) {
+        if (units > 0) {
+            // every load is issued unconditionally (a load under a branch would be waited for at the join): past the
+            // wave's last unit it reads the chunk's last unit again, which is not multiplied
+            auto fetch = [&](long u, Q(&v)[H][NB]) {
+                const long p = p_begin + min(u, units - 1) * UP + 4 * k4;
+#pragma unroll
+                for (int b = 0; b < NB; b++)
+#pragma unroll
+                    for (int h = 0; h < H; h++) v[h][b] = *(const __attribute__((address_space(1))) Q *)(col[b] + p + 16 * h);
+            };
+            Q va[H][NB], vb[H][NB];
+            long u = wave;
+            fetch(u, va);
+            for (; u + W < units; u += 2 * W) {
+                fetch(u + W, vb);
+                multiply(va, all);
+                fetch(u + 2 * W, va);
+                multiply(vb, all);
+            }
+            if (u < units) multiply(va, all);
         }
-        __builtin_amdgcn_wave_barrier();
-        gram_fetch<T, LOADS>(cols, pn, p_end, v);
+        const long pt = p_begin + units * UP;
+        if (pt < p_end && wave == (int)(units % W)) {  // the tail, fewer than UP points: guarded loads
+            Q v[H][NB];
 #pragma unroll
-        for (int kk = 0; kk < G2_S; kk += 4) {
-            const double a0 = sl[r16][kk + k4];
-            const double a1 = sl[16 + r16][kk + k4];
+            for (int b = 0; b < NB; b++)
 #pragma unroll
-            for (int b = 0; b < 4; b++) {
-                if (live[0][b] || live[1][b]) {
-                    const double bv = sl[brow[b]][kk + k4];
-                    if (live[0][b]) acc[0][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, bv, acc[0][b], 0, 0, 0);
-                    if (live[1][b]) acc[1][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, bv, acc[1][b], 0, 0, 0);
-                }
+                for (int h = 0; h < H; h++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const long p = pt + 16 * h + 4 * k4 + j;
+                        v[h][b][j] = p < p_end ? gload(col[b] + p) : T(0);
+                    }
+            multiply(v, all);
+        }
+    };
+    if (SHARE || live == (1u << (RB * CB)) - 1u) run(std::true_type{});
+    else run(std::false_type{});
+    // sum the waves' accumulators in wave order through LDS, one block per pass
+    double *dst = partials + (long)ch * m * q;
+#pragma unroll
+    for (int a = 0; a < RB; a++)
+#pragma unroll
+        for (int b = 0; b < CB; b++) {
+            if (!((live >> (a * CB + b)) & 1u)) continue;  // uniform over the workgroup
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < 4; r++) red[wave][r * 64 + lane] = acc[a][b][r];
+            __syncthreads();
+            if (wave < 4) {  // wave r sums register r
+                double sum = red[0][threadIdx.x];
+#pragma unroll
+                for (int w = 1; w < W; w++) sum += red[w][threadIdx.x];
+                const int i = i0 + a * 16 + k4 + 4 * wave, j = j0 + b * 16 + c16;
+                if (i < m && j < q) dst[(long)i * q + j] = sum;
             }
         }
-        __builtin_amdgcn_wave_barrier();
-    };
-    // stages in pairs (a stage past the chunk holds zeros and adds nothing)
-    for (; p0 < p_end; p0 += 8 * G2_S) {
-        stage(va, p0 + 8 * G2_S);
-        stage(vb, p0 + 12 * G2_S);
-    }
-    // sum the four waves' accumulators in wave order through LDS, one 16 x 64 half (acc[a]) per pass: 16 doubles per
-    // lane per wave
-    double *red = &slab[0][0][0];
-    double *dst = partials + (long)blockIdx.x * m * q;
-    const int jl = lane & 15, ib = lane >> 4;
-#pragma unroll
-    for (int a = 0; a < 2; a++) {
-        __syncthreads();
-        if (wave > 0) {
-#pragma unroll
-            for (int b = 0; b < 4; b++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) red[(((wave - 1) * 16) + (b * 4 + r)) * 64 + lane] = acc[a][b][r];
-        }
-        __syncthreads();
-        if (wave == 0) {
-#pragma unroll
-            for (int b = 0; b < 4; b++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int slot = b * 4 + r;
-                    const double sum = ((acc[a][b][r] + red[(0 * 16 + slot) * 64 + lane]) +
-                                        red[(1 * 16 + slot) * 64 + lane]) + red[(2 * 16 + slot) * 64 + lane];
-                    const int i = i0 + a * 16 + ib + 4 * r, j = j0 + b * 16 + jl;
-                    if (i < m && j < q) dst[(long)i * q + j] = sum;
-                }
-        }
-    }
 }
 
-// sums the per-chunk partials of every output in a fixed order: 4 outputs per workgroup, 64 lanes per output each
-// summing a strided subset of the chunks, then a fixed shuffle tree
-__global__ __launch_bounds__(256) void k_gram_finish(const double *partials, int chunks, int m, int q, double scale,
+// sums the per-chunk partials of every output in a fixed order: 16 consecutive outputs per workgroup (a chunk's 16 are one
+// 128-byte segment), 64 threads per output each summing a strided subset of the chunks, then a fixed tree
+__global__ __launch_bounds__(1024) void k_gram_finish(const double *partials, int chunks, int m, int q, double scale,
                                                       double *G, int sym) {
-    const int lane = threadIdx.x & 63;
+    __shared__ double sh[64][17];
+    const int o16 = threadIdx.x & 15, cl = threadIdx.x >> 4;
     const long mq = (long)m * q;
-    const long out = blockIdx.x * 4L + (threadIdx.x >> 6);
+    const long out = blockIdx.x * 16L + o16;
     // a skipped block's output is summed from its transposed entry (i, j) -> (j, i)
     long src = out;
     if (out < mq) {
@@ -897,25 +863,66 @@ __global__ __launch_bounds__(256) void k_gram_finish(const double *partials, int
         if (gram_mirrored(sym, m, i, j)) src = (long)j * q + i;
     }
     double acc = 0.0;
-    if (out < mq)
-        for (int c = lane; c < chunks; c += 64) acc += partials[(long)c * mq + src];
+    if (out < mq) {
+        int c = cl;
+        for (; c + 3 * 64 < chunks; c += 4 * 64) {  // four loads in flight
+            double v[4];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
-    if (lane == 0 && out < mq) G[out] = acc * scale;
+            for (int u = 0; u < 4; u++) v[u] = partials[(long)(c + 64 * u) * mq + src];
+#pragma unroll
+            for (int u = 0; u < 4; u++) acc += v[u];
+        }
+        for (; c < chunks; c += 64) acc += partials[(long)c * mq + src];
+    }
+    sh[cl][o16] = acc;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        __syncthreads();
+        if (cl < off) sh[cl][o16] += sh[cl + off][o16];
+    }
+    if (cl == 0 && out < mq) G[out] = sh[0][o16] * scale;
 }
 
-// about 768 workgroups in all: three per CU in one round (the 16-load shape fits four per CU; 512 or 1024 measured
-// slower at the LOBPCG shapes of a 95^3 grid)
-static int gram_chunks(int m, int q, long N) {
-    const int blocks = ((m + G2_TI - 1) / G2_TI) * ((q + G2_TJ - 1) / G2_TJ);
-    int chunks = (768 + blocks - 1) / blocks;
-    const long max_chunks = (N + 4 * G2_S - 1) / (4 * G2_S);
-    if (chunks > max_chunks) chunks = (int)max_chunks;
-    if (chunks < 1) chunks = 1;
-    return chunks;
+// The tiling of an m x q product: nr x nc tiles of RB x CB 16 x 16 blocks (the blocks split evenly, at most 3 x 6 in f32
+// or where the one tile shares its operands, else 3 x 4: the accumulators and two units of operands fill 256 registers)
+// and the chunks of points. A product of one shared tile takes one workgroup per CU, 16 waves (4 per SIMD, up to 128
+// registers) or 8; several tiles take two 4-wave workgroups per CU, so that the tiles that S^T S's symmetry empties or
+// thins leave room for others. The partials of one product stay within GRAM_PARTIALS doubles (lira_gram_noalloc's fixed
+// array) whenever one chunk's do.
+struct GramPlan {
+    int RB, CB, nr, nc, H, chunks;
+    bool share;
+    long chunk;
+};
+constexpr long GRAM_PARTIALS = (long)(LIRA_NOALLOC_SCRATCH_BYTES / sizeof(double));
+// sym: U's first m columns are S's
+static GramPlan gram_plan(int m, int q, long N, int esize, bool sym) {
+    GramPlan g;
+    const int R = (m + 15) / 16, C = (q + 15) / 16;
+    g.nr = (R + 2) / 3;
+    g.RB = (R + g.nr - 1) / g.nr;
+    g.nr = (R + g.RB - 1) / g.RB;
+    g.share = sym && g.nr == 1 && C <= 6;  // R <= C, for q >= m
+    const int most = esize == 4 || g.share ? 6 : 4;
+    g.nc = (C + most - 1) / most;
+    g.CB = (C + g.nc - 1) / g.nc;
+    g.nc = (C + g.CB - 1) / g.CB;
+    g.H = esize == 4 && g.RB + g.CB <= 5 ? 2 : 1;
+    long want = std::max(1L, (g.share ? 256L : 512L) / (g.nr * g.nc));
+    want = std::max(1L, std::min(want, GRAM_PARTIALS / ((long)m * q)));
+    const long unit = 16 * g.H;
+    g.chunk = ((N + want - 1) / want + unit - 1) / unit * unit;
+    g.chunks = (int)((N + g.chunk - 1) / g.chunk);
+    return g;
 }
 
-size_t gram_partials_needed(int m, int q, long N) { return (size_t)gram_chunks(m, q, N) * m * q; }
+size_t gram_partials_needed(int m, int q, long N) {
+    // the precisions, and U beginning with S or not, may split a product differently
+    int chunks = 0;
+    for (int esize : {4, 8})
+        for (bool sym : {false, true}) chunks = std::max(chunks, gram_plan(m, q, N, esize, sym).chunks);
+    return (size_t)chunks * m * q;
+}
 
 static ColPtrs to_ptrs(const Cols &c) {
     ColPtrs p{};
@@ -930,43 +937,44 @@ static ColPtrs to_ptrs(const Cols &c) {
     return p;
 }
 
+template <typename T, int RB, int CB, bool SHARE>
+static void launch_gram(const GramPlan &g, const ColPtrs &sp, const ColPtrs &up, int m, int q, long N, double *partials,
+                        int sym, hipStream_t s) {
+    const int total = g.chunks * g.nr * g.nc;
+    const dim3 grid((unsigned)(8 * ((total + 7) / 8)));
+    constexpr bool TWO = sizeof(T) == 4 && RB + CB <= 5;
+    hipLaunchKernelGGL((k_gram<T, RB, CB, SHARE, TWO ? 2 : 1>), grid, dim3(64 * gram_waves(RB, CB, SHARE)), 0, s, sp, up, m, q, N, g.chunk, g.chunks,
+                       g.nc, g.nr * g.nc, partials, sym);
+}
+
 template <typename T>
 void gram(const Cols &S, const Cols &U, long N, double scale, double *partials, size_t partial_cap, double *G,
           hipStream_t s) {
     const int m = S.total(), q = U.total();
     if (m == 0 || q == 0) return;
-    const int chunks = gram_chunks(m, q, N);
-    if ((size_t)chunks * m * q > partial_cap) throw InvalidError("gram: partial buffer too small");
-    long chunk = (N + chunks - 1) / chunks;
-    chunk = ((chunk + 4 * G2_S - 1) / (4 * G2_S)) * (4 * G2_S);
-    const int blocks = ((m + G2_TI - 1) / G2_TI) * ((q + G2_TJ - 1) / G2_TJ);
     // U begins with S's m columns (LOBPCG's U = [S, R, HW, HP]): S^T S is symmetric and its lower blocks are mirrored
     const ColPtrs sp = to_ptrs(S), up = to_ptrs(U);
     int sym = q >= m ? 1 : 0;
     for (int j = 0; j < m && sym; j++)
         if (col_host(sp, j, N, sizeof(T)) != col_host(up, j, N, sizeof(T))) sym = 0;
-    // the packed U columns of the fullest tile: those neither past q nor among the tile's S columns
-    int packed = 0;
-    const int nbi = (m + G2_TI - 1) / G2_TI, nbj = (q + G2_TJ - 1) / G2_TJ;
-    for (int bi = 0; bi < nbi; bi++) {
-        std::vector<const void *> sc;
-        for (int i = bi * G2_TI; i < std::min(m, (bi + 1) * G2_TI); i++) sc.push_back(col_host(sp, i, N, sizeof(T)));
-        for (int bj = 0; bj < nbj; bj++) {
-            int cnt = 0;
-            for (int j = bj * G2_TJ; j < std::min(q, (bj + 1) * G2_TJ); j++)
-                if (std::find(sc.begin(), sc.end(), col_host(up, j, N, sizeof(T))) == sc.end()) cnt++;
-            packed = std::max(packed, cnt);
-        }
+    const GramPlan g = gram_plan(m, q, N, (int)sizeof(T), sym != 0);
+    if ((size_t)g.chunks * m * q > partial_cap) throw InvalidError("gram: partial buffer too small");
+#define LIRA_GRAM(R_, C_)                                                                                              \
+    if (g.RB == R_ && g.CB == C_) {                                                                                    \
+        if constexpr (R_ <= C_) {                                                                                      \
+            if (g.share) launch_gram<T, R_, C_, true>(g, sp, up, m, q, N, partials, sym, s);                             \
+        }                                                                                                              \
+        if constexpr (sizeof(T) == 4 || C_ <= 4) {                                                                     \
+            if (!g.share) launch_gram<T, R_, C_, false>(g, sp, up, m, q, N, partials, sym, s);                           \
+        }                                                                                                              \
     }
-    const int loads = 8 + (packed + 15) / 16 * 4;  // 12, 16, 20 or 24 elements per lane per stage
-    const dim3 grid(chunks, blocks);
-    if (loads <= 12) hipLaunchKernelGGL((k_gram<T, 12>), grid, dim3(256), 0, s, sp, up, m, q, N, chunk, partials, sym);
-    else if (loads <= 16) hipLaunchKernelGGL((k_gram<T, 16>), grid, dim3(256), 0, s, sp, up, m, q, N, chunk, partials, sym);
-    else if (loads <= 20) hipLaunchKernelGGL((k_gram<T, 20>), grid, dim3(256), 0, s, sp, up, m, q, N, chunk, partials, sym);
-    else hipLaunchKernelGGL((k_gram<T, 24>), grid, dim3(256), 0, s, sp, up, m, q, N, chunk, partials, sym);
+    LIRA_GRAM(1, 1) LIRA_GRAM(1, 2) LIRA_GRAM(1, 3) LIRA_GRAM(1, 4) LIRA_GRAM(1, 5) LIRA_GRAM(1, 6)
+    LIRA_GRAM(2, 1) LIRA_GRAM(2, 2) LIRA_GRAM(2, 3) LIRA_GRAM(2, 4) LIRA_GRAM(2, 5) LIRA_GRAM(2, 6)
+    LIRA_GRAM(3, 1) LIRA_GRAM(3, 2) LIRA_GRAM(3, 3) LIRA_GRAM(3, 4) LIRA_GRAM(3, 5) LIRA_GRAM(3, 6)
+#undef LIRA_GRAM
     LIRA_HIP(hipGetLastError());
     const long mq = (long)m * q;
-    hipLaunchKernelGGL(k_gram_finish, dim3((unsigned)((mq + 3) / 4)), dim3(256), 0, s, partials, chunks, m, q, scale, G,
+    hipLaunchKernelGGL(k_gram_finish, dim3((unsigned)((mq + 15) / 16)), dim3(1024), 0, s, partials, g.chunks, m, q, scale, G,
                        sym);
     LIRA_HIP(hipGetLastError());
 }
