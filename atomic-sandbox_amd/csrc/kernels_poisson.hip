@@ -356,102 +356,10 @@ void poisson_rhs(double *b, const T *rho, const double *q, double *ghost, int n,
 // ---------------------------------------------------------------------------------------- multigrid ----
 // Level operator A2 x = (diag x - nb)/H^2 with nb the six in-box neighbours and diag = 6 - (ghost factors of the
 // touched faces) (qm-gpu/src/multigrid.rs:10-26): a missing neighbour at boundary distance d is (1 - 1/d) x0.
-template <typename T>
-__device__ inline void a2_parts(const T *x, int i, int j, int k, int n, T g_low, T g_high, T &nb, T &diag) {
-    const long nn = (long)n * n;
-    const long id = i + (long)n * j + nn * k;
-    T s = T(0), g = T(0);
-    if (i > 0) s += x[id - 1]; else g += g_low;
-    if (i < n - 1) s += x[id + 1]; else g += g_high;
-    if (j > 0) s += x[id - n]; else g += g_low;
-    if (j < n - 1) s += x[id + n]; else g += g_high;
-    if (k > 0) s += x[id - nn]; else g += g_low;
-    if (k < n - 1) s += x[id + nn]; else g += g_high;
-    nb = s;
-    diag = T(6) - g;
-}
-
-// the level operators per point (shared by the per-level kernels and the fused coarse V-cycle, so both compute
-// bitwise the same values)
-template <typename T>
-__device__ inline T mg_jacobi_pt(const T *x, const T *b, long p, int i, int j, int k, int n, T h2, T omega, T g_low,
-                                 T g_high) {
-    T nb, diag;
-    a2_parts(x, i, j, k, n, g_low, g_high, nb, diag);
-    const T xq = x[p];
-    return xq + (omega / diag) * (h2 * b[p] + nb - diag * xq);
-}
-template <typename T>
-__device__ inline T mg_residual_pt(const T *x, const T *b, long p, int i, int j, int k, int n, T h2, T g_low,
-                                   T g_high) {
-    T nb, diag;
-    a2_parts(x, i, j, k, n, g_low, g_high, nb, diag);
-    return b[p] + (nb - diag * x[p]) / h2;
-}
-// full weighting onto coarse point (i, j, k) from the fine point (2i + 1, 2j + 1, 2k + 1) and its 26 neighbours
-template <typename T> __device__ inline T mg_restrict_pt(const T *f, int i, int j, int k, int nf) {
-    const long nff = (long)nf * nf;
-    T s = T(0);
-    for (int dz = -1; dz <= 1; dz++) {
-        const int c = 2 * k + 1 + dz;
-        if (c < 0 || c >= nf) continue;
-        const T wz = dz == 0 ? T(0.5) : T(0.25);
-        for (int dy = -1; dy <= 1; dy++) {
-            const int bb = 2 * j + 1 + dy;
-            if (bb < 0 || bb >= nf) continue;
-            const T wy = dy == 0 ? T(0.5) : T(0.25);
-            for (int dx = -1; dx <= 1; dx++) {
-                const int a = 2 * i + 1 + dx;
-                if (a < 0 || a >= nf) continue;
-                const T wx = dx == 0 ? T(0.5) : T(0.25);
-                s += wx * wy * wz * f[a + (long)nf * bb + nff * c];
-            }
-        }
-    }
-    return s;
-}
-// trilinear interpolation of the coarse correction at fine point (i, j, k): odd fine indices sit on a coarse point,
-// even ones halfway between two
-template <typename T> __device__ inline T mg_prolong_pt(const T *c, int i, int j, int k, int nc) {
-    const long ncc = (long)nc * nc;
-    const int t[3] = {i, j, k};
-    int ci[3][2];
-    T wi[3][2];
-    int cnt[3];
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-        const int cc = t[a] >> 1;
-        if (t[a] & 1) {
-            ci[a][0] = cc;
-            wi[a][0] = T(1);
-            ci[a][1] = -1;
-            wi[a][1] = T(0);
-            cnt[a] = 1;
-        } else {
-            ci[a][0] = cc - 1;
-            wi[a][0] = T(0.5);
-            ci[a][1] = cc;
-            wi[a][1] = T(0.5);
-            cnt[a] = 2;
-        }
-    }
-    T s = T(0);
-    for (int a = 0; a < cnt[0]; a++)
-        for (int b = 0; b < cnt[1]; b++)
-            for (int d = 0; d < cnt[2]; d++) {
-                const int x = ci[0][a], y = ci[1][b], z = ci[2][d];
-                if (x < 0 || y < 0 || z < 0 || x >= nc || y >= nc || z >= nc) continue;
-                s += wi[0][a] * wi[1][b] * wi[2][d] * c[x + (long)nc * y + ncc * z];
-            }
-    return s;
-}
-
 // The per-level kernels of the large levels. One thread per point on a 3-D launch (64 x 4 threads: x fastest, a
 // wave on 64 consecutive points of one row; no index divisions). Every neighbour load is issued unconditionally from a
 // clamped, always valid address and a missing neighbour's term is replaced by an exact zero afterwards, so the loads of
-// a thread are in flight together (a load under a bounds branch made the compiler wait for each in turn). Each sum runs
-// over the same terms in the same order as the per-point functions above (an added exact zero leaves a float sum
-// unchanged), so these kernels produce the values of the fused coarse kernel bit for bit.
+// a thread are in flight together (a load under a bounds branch made the compiler wait for each in turn).
 constexpr int MG_BX = 64, MG_BY = 4;
 inline dim3 mg_grid(int n) { return dim3((unsigned)((n + MG_BX - 1) / MG_BX), (unsigned)((n + MG_BY - 1) / MG_BY), (unsigned)n); }
 
@@ -578,46 +486,9 @@ template <typename T> __global__ __launch_bounds__(256) void k_mg_restrict(T *ds
     dst[i + (long)nc * j + (long)nc * nc * k] = s;
 }
 
-// the trilinear interpolation of the coarse correction at fine point (i, j, k) added in place: per axis an odd fine
-// index sits on coarse point t >> 1 (weight 1), an even one between (t >> 1) - 1 and t >> 1 (1/2 each); the eight
-// terms in the order of mg_prolong_pt, a missing one an exact zero
-template <typename T> __global__ __launch_bounds__(256) void k_mg_prolong_add(T *fine, const T *c, int nf, int nc) {
-    const int i = blockIdx.x * MG_BX + threadIdx.x, j = blockIdx.y * MG_BY + threadIdx.y, k = blockIdx.z;
-    if (i >= nf || j >= nf) return;
-    const long ncc = (long)nc * nc;
-    const int t[3] = {i, j, k};
-    int ci[3][2];
-    T wi[3][2];
-    bool ok[3][2];
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-        const bool odd = t[a] & 1;
-        const int cc = t[a] >> 1;
-        ci[a][0] = odd ? cc : cc - 1;
-        ci[a][1] = cc;
-        wi[a][0] = odd ? T(1) : T(0.5);
-        wi[a][1] = T(0.5);
-        ok[a][0] = ci[a][0] >= 0 && ci[a][0] < nc;
-        ok[a][1] = !odd && cc < nc;  // an odd index has one term
-    }
-    T s = T(0);
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++)
-#pragma unroll
-            for (int d = 0; d < 2; d++) {
-                const bool in = ok[0][a] && ok[1][b] && ok[2][d];
-                const int x = in ? ci[0][a] : 0, y = in ? ci[1][b] : 0, z = in ? ci[2][d] : 0;
-                const T v = c[x + (long)nc * y + ncc * z];
-                s += in ? wi[0][a] * wi[1][b] * wi[2][d] * v : T(0);
-            }
-    fine[i + (long)nf * j + (long)nf * nf * k] += s;
-}
-
 // Restriction with the fine rows read as pairs: coarse point i takes fine 2i, 2i + 1 as one vector load and 2i + 2
 // from its x neighbour's pair (a lane shuffle; the wave's last lane, and the last coarse point, load it). One vector
-// load per fine row instead of three strided ones; the 27 terms in mg_restrict_pt's order. Needs an even fine n (the
+// load per fine row instead of three strided ones. Needs an even fine n (the
 // pairs aligned); every lane stays live for the shuffles and only stores inside the level.
 template <typename T> struct Pair2;
 template <> struct Pair2<float> { typedef float type __attribute__((ext_vector_type(2))); };
@@ -655,7 +526,7 @@ template <typename T> __global__ __launch_bounds__(256) void k_mg_restrict_pairs
 }
 
 // Prolongation-add with one thread per coarse cell: the cell's (up to) 8 fine children 2c + (0, 1) per axis share the
-// 8 coarse values at c - 1 and c, loaded once; each child's terms in mg_prolong_pt's order and weights (an odd fine
+// 8 coarse values at c - 1 and c, loaded once; each child's terms and weights in a fixed order (an odd fine
 // index takes coarse c with weight 1; an even one c - 1 and c with 1/2 each; a missing term an exact zero).
 template <typename T> __global__ __launch_bounds__(256) void k_mg_prolong_cells(T *fine, const T *c, int nf, int nc) {
     const int hx = (nf + 1) / 2;
@@ -692,7 +563,7 @@ template <typename T> __global__ __launch_bounds__(256) void k_mg_prolong_cells(
                 const int i = 2 * cx + sx;
                 if (i >= nf) continue;
                 const int sv[3] = {sx, sy, sz};
-                // per axis the two terms of mg_prolong_pt: (slot, weight, present)
+                // per axis the two terms: (slot, weight, present)
                 int sl[3][2];
                 T wt[3][2];
                 bool in[3][2];
@@ -723,101 +594,209 @@ template <typename T> __global__ __launch_bounds__(256) void k_mg_prolong_cells(
     }
 }
 
-// The V-cycle from a small level down, in one workgroup with every level's x, b and scratch in LDS: the same
-// sequence as the per-level kernels (zero fill, pre-smoothing, residual, restriction, ..., the coarsest sweeps,
-// prolongation, post-smoothing), each pass a loop over the level's points followed by a barrier. Replaces some 25
-// launches per V-cycle whose fixed dispatch cost dominates these tiny grids.
-template <typename T> __global__ __launch_bounds__(1024) void k_mg_coarse(T *x_out, const T *b_in, MgCoarse a) {
+// The V-cycle from a small level down in one workgroup (the same sequence as the per-level kernels: pre-smoothing,
+// residual, restriction, ..., the coarsest sweeps, prolongation, post-smoothing), in place of some 30 launches whose
+// fixed cost is several times their work. A thread owns a z column of a level: its x and b stay in registers, with the z
+// neighbours, and LDS holds one array per level, the x the neighbouring columns read (the residual while the next level
+// restricts it). The arrays have the class's strides (edge NMAX, whatever the level's n: every offset is an immediate) and
+// a zero border (one column after each row, one row after each plane, a plane at either end), so no neighbour read is a
+// branch; a column's diagonal takes three values (first, inner and last plane). Levels of at most 8^2 columns run on the
+// first wave alone, without block barriers. What bounds it is the chain of some 60 LDS latencies and barriers: f64 from
+// 12^3 36.5 -> 14.4 us, f32 from 16^3 50.7 -> 16.1 us (the levels as loops of 1024 threads over all points, every index
+// divided out and every neighbour behind a branch, before). Entering at 24^3 instead (a 576-thread workgroup, 36 us)
+// saved seven launches and took as long as they do (a Hartree solve on 95^3: 3.67 ms against 3.54).
+// one level's LDS array: border, then plane k, row j, point i at (1 + k) (NMAX + 1)^2 + j (NMAX + 1) + i + 1
+static __host__ __device__ constexpr int mgc_level_elems(int nmax) { return (nmax + 1) * (nmax + 1) * (nmax + 2) + 2; }
+// all levels' elements, as a type: a constant in device code too
+template <int NMAX> struct MgcElems {
+    static constexpr int value = mgc_level_elems(NMAX) + MgcElems<(NMAX > 2 ? NMAX / 2 : 0)>::value;
+};
+template <> struct MgcElems<0> {
+    static constexpr int value = 0;
+};
+static constexpr int mgc_threads(int nmax) { return (nmax * nmax + 63) / 64 * 64; }
+
+template <typename T, int NMAX> struct MgcLevel {
+    static constexpr bool WAVE = NMAX * NMAX <= 64;  // one wave owns the level
+    static constexpr int SY = NMAX + 1, SZ = SY * SY;
+    T x[NMAX], b[NMAX];  // b: h^2 times the right-hand side
+    T d0, d1, d2;        // the diagonal on the first, the inner and the last plane
+    T o0, o1, o2;        // omega / diagonal there
+    T h2, inv_h2, rest;
+    T *c;  // the column's first point in LDS
+    int n;
+    bool own;
+
+    __device__ static void sync() {
+        if (WAVE) {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        } else {
+            __syncthreads();
+        }
+    }
+    __device__ static void place(int &i, int &j) {
+        i = (int)threadIdx.x % NMAX;
+        j = (int)threadIdx.x / NMAX;
+    }
+    __device__ void init(const MgCoarse &a, int l, T *lds) {
+        int i, j;
+        place(i, j);
+        n = a.n[l];
+        own = i < n && j < n;
+        h2 = (T)a.h2[l];
+        inv_h2 = T(1) / h2;
+        const T omega = (T)a.omega;
+        rest = T(1) - omega;
+        c = lds + SZ + 1 + (own ? i + SY * j : 0);
+        const T gl = (T)a.gl[l], gh = (T)a.gh[l];
+        T g = T(0);
+        g += i == 0 ? gl : T(0);
+        g += i == n - 1 ? gh : T(0);
+        g += j == 0 ? gl : T(0);
+        g += j == n - 1 ? gh : T(0);
+        d0 = T(6) - (g + gl + (n == 1 ? gh : T(0)));
+        d1 = T(6) - g;
+        d2 = T(6) - (g + gh);
+        o0 = omega / d0;
+        o1 = omega / d1;
+        o2 = omega / d2;
+    }
+    __device__ T diag(int k) const { return k == 0 ? d0 : k == n - 1 ? d2 : d1; }
+    // omega / diagonal, 0 past the level (its x stays 0 there)
+    __device__ T od(int k) const { return k == 0 ? o0 : k < n - 1 ? o1 : k == n - 1 ? o2 : T(0); }
+    __device__ void put(const T (&v)[NMAX]) {  // the column into LDS, between two barriers
+        sync();
+        if (own) {
+#pragma unroll
+            for (int k = 0; k < NMAX; k++) c[SZ * k] = v[k];
+        }
+        sync();
+    }
+    __device__ T around(int k) const { return ((c[SZ * k - 1] + c[SZ * k + 1]) + c[SZ * k - SY]) + c[SZ * k + SY]; }
+    __device__ void sweep0() {  // from x = 0
+#pragma unroll
+        for (int k = 0; k < NMAX; k++) x[k] = od(k) * b[k];
+        put(x);
+    }
+    __device__ void sweep() {
+        T below = T(0);
+#pragma unroll
+        for (int k = 0; k < NMAX; k++) {
+            const T xk = x[k], nb = (around(k) + below) + (k + 1 < NMAX ? x[k + 1] : T(0));
+            x[k] = rest * xk + od(k) * (b[k] + nb);  // x + (omega / d) (h^2 b + nb - d x)
+            below = xk;
+            if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // few neighbour reads in flight at once: registers
+        }
+        put(x);
+    }
+    __device__ void residual() {  // into LDS, in x's place
+        T r[NMAX];
+#pragma unroll
+        for (int k = 0; k < NMAX; k++) {
+            const T nb = (around(k) + (k > 0 ? x[k - 1] : T(0))) + (k + 1 < NMAX ? x[k + 1] : T(0));
+            r[k] = k < n ? inv_h2 * (b[k] + nb - diag(k) * x[k]) : T(0);
+            if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+        put(r);
+    }
+    // b = the full weighting of the finer level's residual (its LDS array f): per fine plane the 9 points about
+    // (2i + 1, 2j + 1), then the three planes about 2k + 1; what lies past the grid is in the zero border
+    template <int NF> __device__ void restrict_from(const T *f) {
+        constexpr int FY = NF + 1, FZ = FY * FY;
+        int i, j;
+        place(i, j);
+        const T *p = f + FZ + 1 + (own ? 2 * i + 1 + FY * (2 * j + 1) : FY + 1);
+        auto plane = [&](int k) {
+            const T *q = p + FZ * k;
+            return T(0.0625) * (((q[-FY - 1] + q[-FY + 1]) + q[FY - 1]) + q[FY + 1]) +
+                   (T(0.125) * (((q[-1] + q[1]) + q[-FY]) + q[FY]) + T(0.25) * q[0]);
+        };
+        T lo = plane(0);
+#pragma unroll
+        for (int k = 0; k < NMAX; k++) {
+            const T mid = plane(2 * k + 1), hi = plane(2 * k + 2);  // plane NF: the border
+            b[k] = k < n ? h2 * (T(0.25) * (lo + hi) + T(0.5) * mid) : T(0);
+            lo = hi;
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    // x += the trilinear interpolation of the coarser level's x (its LDS array f): an odd index sits on coarse t / 2, an
+    // even one between t / 2 - 1 and t / 2
+    template <int NC> __device__ void prolong_from(const T *f) {
+        constexpr int CY = NC + 1, CZ = CY * CY;
+        int i, j;
+        place(i, j);
+        if (!own) i = j = 0;
+        const T *p = f + CZ + 1 + (i >> 1) + CY * (j >> 1);
+        const T wx = i & 1 ? T(0) : T(0.5), wy = j & 1 ? T(0) : T(0.5);
+        auto plane = [&](int k) {
+            const T *q = p + CZ * k;
+            const T lo = wx * q[-CY - 1] + (T(1) - wx) * q[-CY], hi = wx * q[-1] + (T(1) - wx) * q[0];
+            return wy * lo + (T(1) - wy) * hi;
+        };
+        T prev = T(0);
+#pragma unroll
+        for (int k = 0; k < NMAX; k += 2) {
+            const T cur = plane(k / 2);  // plane NC: the border
+            x[k] += k < n ? T(0.5) * (prev + cur) : T(0);
+            if (k + 1 < NMAX) x[k + 1] += k + 1 < n ? cur : T(0);
+            prev = cur;
+            if (k % 8 == 6) __builtin_amdgcn_sched_barrier(0);
+        }
+        put(x);
+    }
+};
+
+// level l of a (at most NMAX points an edge), whose b is in L's registers; on return its x is in registers and LDS
+template <typename T, int NMAX> __device__ __forceinline__ void mgc_cycle(MgcLevel<T, NMAX> &L, const MgCoarse &a, int l, T *lds) {
+    L.sweep0();
+    if (l == a.levels - 1) {
+        for (int s = 1; s < a.coarse; s++) L.sweep();
+        return;
+    }
+    for (int s = 1; s < a.pre; s++) L.sweep();
+    L.residual();
+    if constexpr (NMAX >= 3) {
+        constexpr int NC = NMAX / 2;
+        constexpr int LEVEL = mgc_level_elems(NMAX);
+        T *next = lds + LEVEL;
+        constexpr bool one = MgcLevel<T, NC>::WAVE;
+        if (!one || threadIdx.x < 64) {
+            MgcLevel<T, NC> C;
+            C.init(a, l + 1, next);
+            C.template restrict_from<NMAX>(lds);
+            mgc_cycle<T, NC>(C, a, l + 1, next);
+        }
+        if (one && !L.WAVE) __syncthreads();  // the first wave's x is in LDS
+        L.template prolong_from<NC>(next);
+    }
+    for (int s = 0; s < a.post; s++) L.sweep();
+}
+
+template <typename T, int NMAX>
+__global__ __launch_bounds__(mgc_threads(NMAX)) void k_mg_coarse(T *x_out, const T *b_in, MgCoarse a) {
     extern __shared__ __align__(16) unsigned char mg_smem[];
     T *lds = reinterpret_cast<T *>(mg_smem);
-    const int tid = threadIdx.x;
-    const T omega = (T)a.omega;
-    auto level = [&](int l, T *&x, T *&b, T *&tmp) {
-        const int N = a.n[l] * a.n[l] * a.n[l];
-        x = lds + a.off[l];
-        b = x + N;
-        tmp = b + N;
-    };
-    auto decode = [](int p, int n, int &i, int &j, int &k) {
-        k = p / (n * n);
-        const int rem = p - k * n * n;
-        j = rem / n;
-        i = rem - j * n;
-    };
-    auto smooth = [&](int l, int sweeps) {
-        T *x, *b, *tmp;
-        level(l, x, b, tmp);
-        const int n = a.n[l], N = n * n * n;
-        const T h2 = (T)a.h2[l], gl = (T)a.gl[l], gh = (T)a.gh[l];
-        for (int sw = 0; sw < sweeps; sw += 2) {
-            for (int p = tid; p < N; p += 1024) {
-                int i, j, k;
-                decode(p, n, i, j, k);
-                tmp[p] = mg_jacobi_pt<T>(x, b, p, i, j, k, n, h2, omega, gl, gh);
-            }
-            __syncthreads();
-            for (int p = tid; p < N; p += 1024) {
-                int i, j, k;
-                decode(p, n, i, j, k);
-                x[p] = mg_jacobi_pt<T>(tmp, b, p, i, j, k, n, h2, omega, gl, gh);
-            }
-            __syncthreads();
-        }
-    };
-    {
-        T *x, *b, *tmp;
-        level(0, x, b, tmp);
-        const int N = a.n[0] * a.n[0] * a.n[0];
-        for (int p = tid; p < N; p += 1024) b[p] = b_in[p];
+    MgcLevel<T, NMAX> L;
+    L.init(a, 0, lds);
+    int i, j;
+    L.place(i, j);
+    const int n = L.n, nn = n * n, at = L.own ? i + n * j : 0;
+#pragma unroll
+    for (int k = 0; k < NMAX; k++) {
+        const T v = b_in[at + nn * min(k, n - 1)];
+        L.b[k] = k < n ? L.h2 * v : T(0);
     }
+    constexpr int ELEMS = MgcElems<NMAX>::value, THREADS = mgc_threads(NMAX);
+    for (int e = threadIdx.x; e < ELEMS; e += THREADS) lds[e] = T(0);
     __syncthreads();
-    const int L = a.levels;
-    for (int l = 0; l < L; l++) {
-        T *x, *b, *tmp;
-        level(l, x, b, tmp);
-        const int n = a.n[l], N = n * n * n;
-        for (int p = tid; p < N; p += 1024) x[p] = T(0);
-        __syncthreads();
-        if (l == L - 1) {
-            smooth(l, a.coarse);
-            break;
-        }
-        smooth(l, a.pre);
-        const T h2 = (T)a.h2[l], gl = (T)a.gl[l], gh = (T)a.gh[l];
-        for (int p = tid; p < N; p += 1024) {
-            int i, j, k;
-            decode(p, n, i, j, k);
-            tmp[p] = mg_residual_pt<T>(x, b, p, i, j, k, n, h2, gl, gh);
-        }
-        __syncthreads();
-        T *xc, *bc, *tc;
-        level(l + 1, xc, bc, tc);
-        const int nc = a.n[l + 1], Nc = nc * nc * nc;
-        for (int p = tid; p < Nc; p += 1024) {
-            int i, j, k;
-            decode(p, nc, i, j, k);
-            bc[p] = mg_restrict_pt<T>(tmp, i, j, k, n);
-        }
-        __syncthreads();
-    }
-    for (int l = L - 2; l >= 0; l--) {
-        T *x, *b, *tmp, *xc, *bc, *tc;
-        level(l, x, b, tmp);
-        level(l + 1, xc, bc, tc);
-        const int n = a.n[l], N = n * n * n;
-        for (int p = tid; p < N; p += 1024) {
-            int i, j, k;
-            decode(p, n, i, j, k);
-            x[p] += mg_prolong_pt<T>(xc, i, j, k, a.n[l + 1]);
-        }
-        __syncthreads();
-        smooth(l, a.post);
-    }
-    {
-        T *x, *b, *tmp;
-        level(0, x, b, tmp);
-        const int N = a.n[0] * a.n[0] * a.n[0];
-        for (int p = tid; p < N; p += 1024) x_out[p] = x[p];
+    mgc_cycle<T, NMAX>(L, a, 0, lds);
+    if (L.own) {
+#pragma unroll
+        for (int k = 0; k < NMAX; k++)
+            if (k < n) x_out[at + nn * k] = L.x[k];
     }
 }
 
@@ -865,15 +844,21 @@ void mg_jacobi0(T *dst, const T *b, int n, double h2, double omega, double g_low
                        (T)g_high);
     LIRA_HIP(hipGetLastError());
 }
-// LDS bytes of the fused V-cycle over the levels of a (x, b and scratch per level)
-size_t mg_coarse_bytes(const MgCoarse &a, int esize) {
-    size_t e = 0;
-    for (int l = 0; l < a.levels; l++) e += 3 * (size_t)a.n[l] * a.n[l] * a.n[l];
-    return e * esize;
+template <typename T, int NMAX> static void launch_mg_coarse(T *x, const T *b, const MgCoarse &a, hipStream_t s) {
+    constexpr size_t bytes = MgcElems<NMAX>::value * sizeof(T);
+    static_assert(bytes <= 65536, "the levels must fit the default dynamic LDS");
+    hipLaunchKernelGGL((k_mg_coarse<T, NMAX>), dim3(1), dim3(mgc_threads(NMAX)), bytes, s, x, b, a);
+    LIRA_HIP(hipGetLastError());
 }
 template <typename T> void mg_coarse(T *x, const T *b, const MgCoarse &a, hipStream_t s) {
-    hipLaunchKernelGGL(k_mg_coarse<T>, dim3(1), dim3(1024), mg_coarse_bytes(a, (int)sizeof(T)), s, x, b, a);
-    LIRA_HIP(hipGetLastError());
+    const int n = a.n[0];
+    if (a.levels < 1 || a.levels > MG_MAX_LEVELS || n > MG_COARSE_MAX || a.n[a.levels - 1] > 2 || a.pre < 1 || a.coarse < 1)
+        throw InvalidError("mg_coarse: bad levels");
+    for (int l = 1; l < a.levels; l++)
+        if (a.n[l] != a.n[l - 1] / 2 || a.n[l] < 1) throw InvalidError("mg_coarse: bad levels");
+    if (n <= 6) launch_mg_coarse<T, 6>(x, b, a, s);
+    else if (n <= 12) launch_mg_coarse<T, 12>(x, b, a, s);
+    else launch_mg_coarse<T, MG_COARSE_MAX>(x, b, a, s);
 }
 
 // ------------------------------------------------------------------------------------ CG on device ----

@@ -260,12 +260,10 @@ struct MgCoarse {
     int levels;
     int n[MG_MAX_LEVELS];
     double h2[MG_MAX_LEVELS], gl[MG_MAX_LEVELS], gh[MG_MAX_LEVELS];
-    int off[MG_MAX_LEVELS];  // element offset of each level's x, b, scratch block in LDS
     int pre, post, coarse;
     double omega;
 };
-size_t mg_coarse_bytes(const MgCoarse &a, int esize);
-constexpr size_t MG_COARSE_LDS = 65536;  // the fused levels' LDS budget (the default dynamic LDS limit)
+constexpr int MG_COARSE_MAX = 16;  // the largest edge of the fused levels
 template <typename T> void mg_coarse(T *x, const T *b, const MgCoarse &a, hipStream_t s);
 // device-side CG scalar updates
 // x += (num/den) p ; r -= (num/den) q    (alpha = sc[ia]/sc[ib])

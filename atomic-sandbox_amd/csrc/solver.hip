@@ -937,26 +937,23 @@ template <typename T> void Solver<T>::poisson_setup() {
         c.tmp.alloc(bytes);
         levels_.push_back(std::move(c));
     }
-    // the finest level from which every coarser level fits the fused kernel's LDS budget
+    // the finest level that the fused kernel takes
     mg_entry_ = (int)levels_.size();
     for (int l = (int)levels_.size() - 1; l >= 0 && (int)levels_.size() - l <= MG_MAX_LEVELS; l--) {
         MgCoarse a{};
         a.levels = (int)levels_.size() - l;
-        int off = 0;
         for (int q = 0; q < a.levels; q++) {
             const Level &L = levels_[l + q];
             a.n[q] = L.n;
             a.h2[q] = L.h * L.h;
             a.gl[q] = 1.0 - 1.0 / L.d_low;
             a.gh[q] = 1.0 - 1.0 / L.d_high;
-            a.off[q] = off;
-            off += 3 * L.n * L.n * L.n;
         }
         a.pre = MG_PRE;
         a.post = MG_POST;
         a.coarse = MG_COARSE;
         a.omega = MG_OMEGA;
-        if (mg_coarse_bytes(a, (int)sizeof(T)) > MG_COARSE_LDS) break;
+        if (a.n[0] > MG_COARSE_MAX) break;
         mg_entry_ = l;
         mgc_ = a;
     }
