@@ -268,22 +268,101 @@ __device__ inline void block_sum_rows(double *acc, int rows, double (*lds)[RMAX]
     __syncthreads();
 }
 
+// V_NL is two launches, both bound by latency on a molecule's boxes: what counts is how many loads are in flight and
+// how many blocks a box makes. Both cut an ion's box into the same chunks of 256 * ppt consecutive box points, ppt
+// points to a thread. ppt is the largest of 1..8 that still gives 256 blocks per band group over all ions (one ion of
+// 22^3 points: ppt 1, 42 chunks). It depends on the boxes alone, so a band's sums have the same order whatever block
+// of bands it is in.
+// Water's blocks at 95^3 (one ion of 4 rows, 8 to 16 bands, f32), the projections, their sums and the scatter: 28.7 us
+// as three launches with chunks of 2048 points and a branch at each row, 9.2 us as it is (4.7 and 4.5).
+constexpr int NL_BLOCK = 256, NL_BANDS = 4, NL_MAX_PPT = 8, NL_MIN_BLOCKS = 256;
+static_assert(NL_BANDS * NL_MAX_ROWS <= 64, "one lane of a wave ends with one (band, row) sum");
+
+static int nl_ppt(long max_pts, int nions) {
+    int ppt = NL_MAX_PPT;
+    while (ppt > 1 && (max_pts + (long)NL_BLOCK * ppt - 1) / ((long)NL_BLOCK * ppt) * nions < NL_MIN_BLOCKS) ppt--;
+    return ppt;
+}
+
+int nl_project_chunks(long max_pts, int nions) {
+    const long c = (long)NL_BLOCK * nl_ppt(max_pts, nions);
+    return (int)std::max(1L, (max_pts + c - 1) / c);
+}
+
+// box point q of an ion -> grid index
+__device__ inline long nl_grid_index(const NlIon &ion, int q, int n) {
+    const int t = q / ion.dim[0], px = q - t * ion.dim[0];
+    const int pz = t / ion.dim[1], py = t - pz * ion.dim[1];
+    return (ion.lo[0] + px) + (long)n * ((ion.lo[1] + py) + (long)n * (ion.lo[2] + pz));
+}
+
+// One step of the sum of V values over a wave's lanes: lanes with bit OFF keep the upper half of the values and send
+// the lower, the others the reverse, so V values cost V shuffles in all instead of 6 V. After the step to OFF = 1 lane
+// l holds in v[0] the whole sum of value `first`, if `left` > 0.
+template <int V, int OFF> __device__ inline void wave_sums(double *v, int &first, int &left) {
+    constexpr int H = (V + 1) / 2;
+    const bool up = (threadIdx.x & OFF) != 0;
+#pragma unroll
+    for (int i = 0; i < H; i++) {
+        const double hi = H + i < V ? v[H + i < V ? H + i : i] : 0.0;
+        const double send = up ? v[i] : hi;
+        v[i] = (up ? hi : v[i]) + __shfl_xor(send, OFF, 64);
+    }
+    first += up ? H : 0;
+    left = up ? left - H : (left < H ? left : H);
+    if constexpr (OFF > 1) wave_sums<H, OFF / 2>(v, first, left);
+}
+
+// The sums of one block's chunk for NL_BANDS bands and R >= rows rows (rows past the ion's read its last row again and
+// are not written). Loads carry no branch: points past the box read its last point with weight 0.
+template <typename T, int R>
+__device__ inline void nl_chunk_sums(const NlIon &ion, const T *const *xb, const T *bb, int n, int ppt, int nb, int b0,
+                                     int bands, int chunks, double (*lds)[NL_BANDS * NL_MAX_ROWS], double *P) {
+    const int rows = ion.rows, pts = (int)ion.pts;
+    double acc[NL_BANDS * R];
+#pragma unroll
+    for (int i = 0; i < NL_BANDS * R; i++) acc[i] = 0.0;
+    const int p0 = (int)blockIdx.x * NL_BLOCK * ppt + (int)threadIdx.x;
+#pragma unroll 2
+    for (int k = 0; k < ppt; k++) {
+        const int p = p0 + k * NL_BLOCK;
+        const bool in = p < pts;
+        const int q = in ? p : pts - 1;
+        const double w = in ? 1.0 : 0.0;
+        T bv[R], xv[NL_BANDS];
+#pragma unroll
+        for (int r = 0; r < R; r++) bv[r] = bb[(long)(r < rows ? r : rows - 1) * pts + q];
+        const long g = nl_grid_index(ion, q, n);
+#pragma unroll
+        for (int j = 0; j < NL_BANDS; j++) xv[j] = xb[j][g];
+#pragma unroll
+        for (int j = 0; j < NL_BANDS; j++) {
+            const double x = w * (double)xv[j];
+#pragma unroll
+            for (int r = 0; r < R; r++) acc[j * R + r] += (double)bv[r] * x;
+        }
+    }
+    int first = 0, left = NL_BANDS * R;
+    wave_sums<NL_BANDS * R, 32>(acc, first, left);
+    if (left > 0) lds[threadIdx.x >> 6][first] = acc[0];
+    __syncthreads();
+    const int i = threadIdx.x, j = i / R, r = i - j * R;
+    if (i < NL_BANDS * R && j < bands && r < rows)
+        P[((long)(ion.row_off + r) * nb + b0 + j) * chunks + blockIdx.x] =
+            ((lds[0][i] + lds[1][i]) + lds[2][i]) + lds[3][i];
+}
+
 // Projections over chunks of each ion's box. Block (chunk, ion, band group) writes the partial sums of its chunk for
-// NL_BANDS bands, P[((row_off + r) * nb + b) * chunks + chunk] = sum over the chunk's points of beta_r(p) x_b(p) (a
-// chunk is NL_CHUNK consecutive box points, 8 per thread; chunks past an ion's box write zeros); k_nl_finish then sums
-// each (row, band)'s chunks in a fixed order into C[(row_off + r) * nb + b] = dv * sum. Bands b < n1 read x1, the
-// others x2 (two blocks in one launch). (Folding the finish into the last chunk block to arrive costs more: each
-// block would pay a device-scope release fence, a write-back of its XCD's dirty L2 lines.)
-constexpr int NL_CHUNK = 2048, NL_BANDS = 4;
+// NL_BANDS bands, P[((row_off + r) * nb + b) * chunks + chunk] = sum over the chunk's points of beta_r(p) x_b(p)
+// (a box has at least one point; chunks past an ion's box write zeros). Bands b < n1 read x1, the others x2 (two blocks in one launch).
 template <typename T>
-__global__ __launch_bounds__(256) void k_nl_project(const T *x1, int n1, const T *x2, int nb, long N, int n,
-                                                    const T *beta, const NlIon *ions, int chunks, double *P) {
-    __shared__ double lds[4][NL_MAX_ROWS];
+__global__ __launch_bounds__(NL_BLOCK) void k_nl_project(const T *x1, int n1, const T *x2, int nb, long N, int n,
+                                                         const T *beta, const NlIon *ions, int ppt, int chunks,
+                                                         double *P) {
+    __shared__ double lds[NL_BLOCK / 64][NL_BANDS * NL_MAX_ROWS];
     const NlIon &ion = ions[blockIdx.y];
-    const int b0 = blockIdx.z * NL_BANDS, chunk = blockIdx.x;
+    const int b0 = blockIdx.z * NL_BANDS;
     const int bands = nb - b0 < NL_BANDS ? nb - b0 : NL_BANDS;
-    const int rows = ion.rows;
-    const int pts = (int)ion.pts, dx = ion.dim[0], dy = ion.dim[1];
     const T *xb[NL_BANDS];
 #pragma unroll
     for (int j = 0; j < NL_BANDS; j++) {
@@ -291,107 +370,118 @@ __global__ __launch_bounds__(256) void k_nl_project(const T *x1, int n1, const T
         xb[j] = b < n1 ? x1 + (long)b * N : x2 + (long)(b - n1) * N;
     }
     const T *bb = beta + ion.beta_off;
-    double acc[NL_BANDS][NL_MAX_ROWS];
-#pragma unroll
-    for (int j = 0; j < NL_BANDS; j++)
-#pragma unroll
-        for (int r = 0; r < NL_MAX_ROWS; r++) acc[j][r] = 0.0;
-    const int p0 = chunk * NL_CHUNK + (int)threadIdx.x;
-    // points past the box read the box's last point with weight 0: the loads carry no branch, so the unrolled
-    // iterations issue them together
-#pragma unroll 4
-    for (int k = 0; k < (pts > 0 ? NL_CHUNK / 256 : 0); k++) {
-        const int p = p0 + k * 256;
-        const bool in = p < pts;
-        const int q = in ? p : pts - 1;
-        const double w = in ? 1.0 : 0.0;
-        const int px = q % dx, t = q / dx;
-        const int py = t % dy, pz = t / dy;
-        const long g = (ion.lo[0] + px) + (long)n * ((ion.lo[1] + py) + (long)n * (ion.lo[2] + pz));
-        double xv[NL_BANDS];
-#pragma unroll
-        for (int j = 0; j < NL_BANDS; j++) xv[j] = w * (double)xb[j][g];
-#pragma unroll
-        for (int r = 0; r < NL_MAX_ROWS; r++)
-            if (r < rows) {
-                const double bv = (double)bb[(long)r * pts + q];
-#pragma unroll
-                for (int j = 0; j < NL_BANDS; j++) acc[j][r] += bv * xv[j];
-            }
-    }
-#pragma unroll
-    for (int j = 0; j < NL_BANDS; j++) {
-        if (j < bands) {  // uniform over the block
-            block_sum_rows<NL_MAX_ROWS>(acc[j], rows, lds);
-            if ((int)threadIdx.x < rows) {
-                const int r = threadIdx.x;
-                P[((long)(ion.row_off + r) * nb + b0 + j) * chunks + chunk] =
-                    ((lds[0][r] + lds[1][r]) + lds[2][r]) + lds[3][r];
-            }
-            __syncthreads();
-        }
-    }
+    if (ion.rows <= 4)  // uniform over the block
+        nl_chunk_sums<T, 4>(ion, xb, bb, n, ppt, nb, b0, bands, chunks, lds, P);
+    else
+        nl_chunk_sums<T, NL_MAX_ROWS>(ion, xb, bb, n, ppt, nb, b0, bands, chunks, lds, P);
 }
 
-// C[pair] = dv * the sum of P[pair * chunks + c] over the chunks, pair = row * nb + band, one wave per pair: lane l
-// sums chunks l, l + 64, ... in order, then the wave's fixed shuffle tree
-__global__ __launch_bounds__(256) void k_nl_finish(const double *P, int chunks, long pairs, double dv, double *C) {
-    const int lane = threadIdx.x & 63;
-    const long pair = blockIdx.x * 4L + (threadIdx.x >> 6);
-    if (pair >= pairs) return;  // uniform over the wave
-    const double *pp = P + pair * chunks;
+// one wave: the sum of a (row, band)'s chunk partials, lane l taking chunks l, l + 64, ... in order, then a fixed
+// shuffle tree; valid in lane 0
+__device__ inline double nl_sum_chunks(const double *pp, int chunks) {
     double v = 0.0;
-    for (int c = lane; c < chunks; c += 64) v += pp[c];
+    for (int c = threadIdx.x & 63; c < chunks; c += 64) v += pp[c];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-    if (lane == 0) C[pair] = dv * v;
+    return v;
 }
 
-// out_b(p) += sum_r E_r C[r][b] beta_r(p) over the boxes of the ions of one colour (disjoint boxes: no two threads
-// touch one point); blockIdx.y picks the ion of the colour, blockIdx.z the band (b < n1 in out1, the rest in out2)
-template <typename T>
-__global__ __launch_bounds__(256) void k_nl_apply(T *out1, int n1, T *out2, int nb, long N, int n, const T *beta,
-                                                  const NlIon *ions, const int *members, const double *C,
-                                                  const double *erow) {
-    const NlIon &ion = ions[members[blockIdx.y]];
-    const long p = blockIdx.x * 256L + threadIdx.x;
-    if (p >= ion.pts) return;
-    const int b = blockIdx.z;
-    const long px = p % ion.dim[0], t = p / ion.dim[0];
-    const long py = t % ion.dim[1], pz = t / ion.dim[1];
-    const long g = (ion.lo[0] + px) + (long)n * ((ion.lo[1] + py) + (long)n * (ion.lo[2] + pz));
-    double acc = 0.0;
-    for (int r = 0; r < ion.rows; r++) {
+// C[pair] = dv * the sum of P[pair * chunks + c] over the chunks, pair = row * nb + band, one wave per pair
+__global__ __launch_bounds__(256) void k_nl_finish(const double *P, int chunks, long pairs, double dv, double *C) {
+    const long pair = blockIdx.x * 4L + (threadIdx.x >> 6);
+    if (pair >= pairs) return;  // uniform over the wave
+    const double v = nl_sum_chunks(P + pair * chunks, chunks);
+    if ((threadIdx.x & 63) == 0) C[pair] = dv * v;
+}
+
+// the points of one block's chunk, out(p) += sum_r ec_r beta_r(p); the first point's loads are issued before the
+// block's waves sum the ion's C (as k_nl_finish does, so both give the same C), which chunk 0 writes
+template <typename T, int R>
+__device__ inline void nl_chunk_apply(const NlIon &ion, T *ob, const T *bb, int n, int ppt, int nb, int b, int chunks,
+                                      const double *P, double dv, double *C, const double *erow, double *ec) {
+    const int rows = ion.rows, pts = (int)ion.pts;
+    int p = (int)blockIdx.x * NL_BLOCK * ppt + (int)threadIdx.x;
+    T bv[R], ov = T(0);
+    long g = 0;
+    auto load = [&] {
+        const int q = p < pts ? p : pts - 1;
+#pragma unroll
+        for (int r = 0; r < R; r++) bv[r] = bb[(long)(r < rows ? r : rows - 1) * pts + q];
+        g = nl_grid_index(ion, q, n);
+        ov = ob[g];
+    };
+    load();
+    for (int r = threadIdx.x >> 6; r < rows; r += NL_BLOCK / 64) {
         const long row = ion.row_off + r;
-        acc += erow[row] * C[row * nb + b] * (double)beta[ion.beta_off + (long)r * ion.pts + p];
+        const double c = dv * nl_sum_chunks(P + (row * nb + b) * chunks, chunks);
+        if ((threadIdx.x & 63) == 0) {
+            ec[r] = erow[row] * c;
+            if (blockIdx.x == 0) C[row * nb + b] = c;
+        }
     }
-    T *ob = b < n1 ? out1 + (long)b * N : out2 + (long)(b - n1) * N;
-    ob[g] = (T)((double)ob[g] + acc);
+    __syncthreads();
+    for (int k = 0; k < ppt && p < pts; k++) {
+        double acc = 0.0;
+#pragma unroll
+        for (int r = 0; r < R; r++)
+            if (r < rows) acc += ec[r] * (double)bv[r];
+        ob[g] = (T)((double)ov + acc);
+        p += NL_BLOCK;
+        if (k + 1 < ppt) load();
+    }
 }
 
-int nl_project_chunks(long max_pts) { return (int)std::max(1L, (max_pts + NL_CHUNK - 1) / NL_CHUNK); }
+// C[r][b] = dv * the sum of its chunk partials, and out_b(p) += sum_r E_r C[r][b] beta_r(p) over the boxes of the ions
+// of one colour (disjoint boxes: no two threads touch one point); blockIdx.y picks the ion of the colour, blockIdx.z
+// the band (b < n1 in out1, the rest in out2). Each block sums its own C again: the partials of one band are
+// chunks / (128 ppt) of the f32 beta that the block reads, and a launch in between costs more. (Summing in the last
+// chunk block to arrive costs more too: each block would pay a device-scope release fence, a write-back of its XCD's
+// dirty L2 lines.)
+template <typename T>
+__global__ __launch_bounds__(NL_BLOCK) void k_nl_apply(T *out1, int n1, T *out2, int nb, long N, int n, const T *beta,
+                                                       const NlIon *ions, const int *members, int ppt, int chunks,
+                                                       const double *P, double dv, double *C, const double *erow) {
+    __shared__ double ec[NL_MAX_ROWS];
+    const NlIon &ion = ions[members[blockIdx.y]];
+    // a chunk past the ion's box has no points; chunk 0 writes C all the same
+    if (blockIdx.x > 0 && (long)blockIdx.x * NL_BLOCK * ppt >= ion.pts) return;  // uniform over the block
+    const int b = blockIdx.z;
+    T *ob = b < n1 ? out1 + (long)b * N : out2 + (long)(b - n1) * N;
+    const T *bb = beta + ion.beta_off;
+    if (ion.rows <= 4)  // uniform over the block
+        nl_chunk_apply<T, 4>(ion, ob, bb, n, ppt, nb, b, chunks, P, dv, C, erow, ec);
+    else
+        nl_chunk_apply<T, NL_MAX_ROWS>(ion, ob, bb, n, ppt, nb, b, chunks, P, dv, C, erow, ec);
+}
 
 template <typename T>
 void nl_project(const T *x1, int n1, const T *x2, int n2, long N, int n, const T *beta, const NlIon *ions, int nions,
-                long max_pts, int rows, double dv, double *C, double *work, hipStream_t s) {
+                long max_pts, double *work, hipStream_t s) {
     const int nb = n1 + n2;
     if (nions <= 0 || nb <= 0) return;
-    const int chunks = nl_project_chunks(max_pts);
-    hipLaunchKernelGGL(k_nl_project<T>, dim3(chunks, nions, (nb + NL_BANDS - 1) / NL_BANDS), dim3(256), 0, s, x1, n1,
-                       x2, nb, N, n, beta, ions, chunks, work);
+    const int chunks = nl_project_chunks(max_pts, nions);
+    hipLaunchKernelGGL(k_nl_project<T>, dim3(chunks, nions, (nb + NL_BANDS - 1) / NL_BANDS), dim3(NL_BLOCK), 0, s, x1,
+                       n1, x2, nb, N, n, beta, ions, nl_ppt(max_pts, nions), chunks, work);
     LIRA_HIP(hipGetLastError());
+}
+
+void nl_finish(const double *work, int nb, int nions, long max_pts, int rows, double dv, double *C, hipStream_t s) {
+    if (nions <= 0 || nb <= 0) return;
     const long pairs = (long)rows * nb;
-    hipLaunchKernelGGL(k_nl_finish, dim3((unsigned)((pairs + 3) / 4)), dim3(256), 0, s, work, chunks, pairs, dv, C);
+    hipLaunchKernelGGL(k_nl_finish, dim3((unsigned)((pairs + 3) / 4)), dim3(256), 0, s, work,
+                       nl_project_chunks(max_pts, nions), pairs, dv, C);
     LIRA_HIP(hipGetLastError());
 }
 
 template <typename T>
-void nl_apply(T *out1, int n1, T *out2, int n2, long N, int n, const T *beta, const NlIon *ions, const int *members,
-              int nmembers, long max_pts, const double *C, const double *erow, hipStream_t s) {
+void nl_apply(T *out1, int n1, T *out2, int n2, long N, int n, const T *beta, const NlIon *ions, int nions,
+              long max_pts, const int *members, int nmembers, const double *work, double dv, double *C,
+              const double *erow, hipStream_t s) {
     const int nb = n1 + n2;
-    if (nmembers <= 0 || nb <= 0 || max_pts <= 0) return;
-    hipLaunchKernelGGL(k_nl_apply<T>, dim3((unsigned)((max_pts + 255) / 256), nmembers, nb), dim3(256), 0, s, out1, n1,
-                       out2, nb, N, n, beta, ions, members, C, erow);
+    if (nmembers <= 0 || nb <= 0) return;
+    const int chunks = nl_project_chunks(max_pts, nions);
+    hipLaunchKernelGGL(k_nl_apply<T>, dim3(chunks, nmembers, nb), dim3(NL_BLOCK), 0, s, out1, n1, out2, nb, N, n, beta,
+                       ions, members, nl_ppt(max_pts, nions), chunks, work, dv, C, erow);
     LIRA_HIP(hipGetLastError());
 }
 
@@ -553,10 +643,10 @@ void nl_force(const T *psi, int nb, long N, int n, double h, const NlIon *ions, 
                                   double, hipStream_t);                                                               \
     template void ionic_fields<T>(T *, T *, int, double, const IonicCentre *, int, const double *, hipStream_t);      \
     template void nl_beta<T>(T *, const NlIon &, int, double, const double *, hipStream_t);                          \
-    template void nl_project<T>(const T *, int, const T *, int, long, int, const T *, const NlIon *, int, long, int,  \
-                                double, double *, double *, hipStream_t);                                             \
-    template void nl_apply<T>(T *, int, T *, int, long, int, const T *, const NlIon *, const int *, int, long,          \
-                              const double *, const double *, hipStream_t);                                           \
+    template void nl_project<T>(const T *, int, const T *, int, long, int, const T *, const NlIon *, int, long,       \
+                                double *, hipStream_t);                                                               \
+    template void nl_apply<T>(T *, int, T *, int, long, int, const T *, const NlIon *, int, long, const int *, int,   \
+                              const double *, double, double *, const double *, hipStream_t);                         \
     template void ionic_forces<T>(const T *, const T *, const T *, int, double, const IonicCentre *, const double *, \
                                   int, double *, double *, hipStream_t);                                              \
     template void nl_force<T>(const T *, int, long, int, double, const NlIon *, int, const double *, double *,       \

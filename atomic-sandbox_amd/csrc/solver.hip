@@ -633,7 +633,6 @@ template <typename T> class Solver final : public SolverIface {
     std::vector<double> nl_e_h_;
     struct Colour {
         int off, count;
-        long max_pts;
     };
     std::vector<Colour> colours_;
     int nl_rows_ = 0;
@@ -660,7 +659,8 @@ template <typename T> class Solver final : public SolverIface {
     }
     void ionic_geometry(double sigma);
     void nl_apply_block(const T *x, T *out, int nb, const T *x2 = nullptr, T *out2 = nullptr, int nb2 = 0);
-    void nl_projections(const T *x, int nb, const T *x2 = nullptr, int nb2 = 0);
+    void nl_projections(const T *x, int nb);
+    long nl_max_pts() const;
     void ensure_nl(int nb);  // the projections' buffers for nb bands
     std::vector<double> nl_energy_terms(Channel<T> &c, bool fd);
 
@@ -1863,11 +1863,8 @@ template <typename T> void Solver<T>::ionic_geometry(double sigma) {
     }
     std::vector<int> members;
     for (auto &g : groups) {
-        Colour c{(int)members.size(), (int)g.size(), 0};
-        for (int i : g) {
-            members.push_back(i);
-            c.max_pts = std::max(c.max_pts, nl_h_[i].pts);
-        }
+        Colour c{(int)members.size(), (int)g.size()};
+        members.insert(members.end(), g.begin(), g.end());
         colours_.push_back(c);
     }
     if (nl_ions_.bytes < nl_h_.size() * sizeof(NlIon)) nl_ions_.alloc(nl_h_.size() * sizeof(NlIon));
@@ -1887,28 +1884,36 @@ template <typename T> void Solver<T>::ensure_nl(int nb) {
         nl_C_.alloc(need * sizeof(double));
         nl_C_cap_ = need;
     }
-    long max_pts = 0;
-    for (const NlIon &ion : nl_h_) max_pts = std::max(max_pts, ion.pts);
-    const size_t work = (size_t)nl_rows_ * nb * nl_project_chunks(max_pts);
+    const size_t work = (size_t)nl_rows_ * nb * nl_project_chunks(nl_max_pts(), (int)nl_h_.size());
     if (work > nl_P_cap_) {
         nl_P_.alloc(work * sizeof(double));
         nl_P_cap_ = work;
     }
 }
 
-template <typename T> void Solver<T>::nl_projections(const T *x, int n1, const T *x2, int n2) {
-    ensure_nl(n1 + n2);
-    long max_pts = 0;
-    for (const NlIon &ion : nl_h_) max_pts = std::max(max_pts, ion.pts);
-    nl_project<T>(x, n1, x2, n2, N_, n_, beta_.template as<T>(), nl_ions_.as<NlIon>(), (int)nl_h_.size(), max_pts,
-                  nl_rows_, dv_, nl_C_.as<double>(), nl_P_.as<double>(), stream_);
+template <typename T> long Solver<T>::nl_max_pts() const {
+    long m = 0;
+    for (const NlIon &ion : nl_h_) m = std::max(m, ion.pts);
+    return m;
+}
+
+template <typename T> void Solver<T>::nl_projections(const T *x, int nb) {
+    ensure_nl(nb);
+    nl_project<T>(x, nb, nullptr, 0, N_, n_, beta_.template as<T>(), nl_ions_.as<NlIon>(), (int)nl_h_.size(),
+                  nl_max_pts(), nl_P_.as<double>(), stream_);
+    nl_finish(nl_P_.as<double>(), nb, (int)nl_h_.size(), nl_max_pts(), nl_rows_, dv_, nl_C_.as<double>(), stream_);
 }
 
 template <typename T> void Solver<T>::nl_apply_block(const T *x, T *out, int nb, const T *x2, T *out2, int nb2) {
-    nl_projections(x, nb, x2, nb2);
+    ensure_nl(nb + nb2);
+    const int nions = (int)nl_h_.size();
+    const long max_pts = nl_max_pts();
+    nl_project<T>(x, nb, x2, nb2, N_, n_, beta_.template as<T>(), nl_ions_.as<NlIon>(), nions, max_pts,
+                  nl_P_.as<double>(), stream_);
     for (const Colour &c : colours_)
-        nl_apply<T>(out, nb, out2, nb2, N_, n_, beta_.template as<T>(), nl_ions_.as<NlIon>(),
-                    nl_members_.as<int>() + c.off, c.count, c.max_pts, nl_C_.as<double>(), nl_erow_.as<double>(), stream_);
+        nl_apply<T>(out, nb, out2, nb2, N_, n_, beta_.template as<T>(), nl_ions_.as<NlIon>(), nions, max_pts,
+                    nl_members_.as<int>() + c.off, c.count, nl_P_.as<double>(), dv_, nl_C_.as<double>(),
+                    nl_erow_.as<double>(), stream_);
 }
 
 // E_NL terms f_b E_r c_rb^2 of a channel in (orbital, sphere, m) order; Aufbau: every orbital at f = 1
