@@ -1189,8 +1189,9 @@ template <typename Td, typename Ts> void convert(Td *out, const Ts *a, long N, h
 // with the roots, logarithms and quotients in the forms that they need. The kernel is bound by f64 issue (4 cycles per
 // instruction and wave): with the library's cbrt, log and sqrt and IEEE division a point took 664 f64 instructions, here
 // 273. Each form starts from a hardware estimate and ends with one step of third order, whose last operation is an fma:
-// relative errors below 1 ulp. 95^3 f32: 23.5 -> 11.9 us a call; the f64 kernel alone 27.6 -> 14.3 us. Against 50-digit
-// arithmetic the errors equal exc_point's (n of 1e-19 .. 1e5: both are set by the rounding of 1 + 1 / q1).
+// relative errors below 1 ulp. 95^3 f32: 23.5 -> 11.8 us a call; the f64 kernel alone 27.6 -> 14.3 us. Mean errors against
+// 113-bit arithmetic over n of 1e-2 .. 1e5, in units of 2^-53, here and with exc_point's forms: e 0.76 and 0.81, v_up 1.32
+// and 1.32, v_down 0.76 and 0.76; at low densities both are set by the rounding of 1 + 1 / q1.
 
 // 1/x: y (1 + e + e^2), e = 1 - x y (the estimates of this and the next are good to some 2^-24)
 __device__ inline double rcp64(double x) {
@@ -1286,8 +1287,9 @@ __device__ inline void lsda_point(double nu, double nd, double &e, double &vu, d
     pw92_point(rs, srs, isr, 0.016887, 0.11125, 10.357, 3.6231, 0.88026, 0.49671, mac, dmac);
     const double ac = -mac, dac = -dmac;
     const double opz = cbrt_unit(1.0 + z), omz = cbrt_unit(1.0 - z);
-    const double f = ((1.0 + z) * opz + (1.0 - z) * omz - 2.0) * 1.9236610509315364;  // 1 / (2^{4/3} - 2)
-    const double fp = 2.564881401242048 * (opz - omz);                                // 4/3 of that
+    const double f0 = (1.0 + z) * opz + (1.0 - z) * omz - 2.0;
+    const double f = fma(f0, 1.9236610509315364, f0 * -6.729470784749165e-17);  // f0 / (2^{4/3} - 2), the constant to 100 bits
+    const double fp = 2.564881401242048 * (opz - omz);  // 4/3 (opz - omz) / (2^{4/3} - 2)
     const double IFPP0 = 1.0 / 1.709921;
     const double z3 = z * z * z, z4 = z3 * z;
     const double ec = ec0 + ac * f * IFPP0 * (1.0 - z4) + (ec1 - ec0) * f * z4;
