@@ -1090,28 +1090,62 @@ template <typename T> void residual(T *r, const T *hx, const T *x, const double 
     LIRA_HIP(hipGetLastError());
 }
 
-// R = HX - theta X and the preconditioner's first pass W = R / max(diag_t + V - lam, 0.1) in one pass (the same
-// per-point formulas as k_residual and k_precond_init)
+// R = HX - theta X, the preconditioner's first pass W = R / max(diag_t + V - lam, 0.1) and the partial sums of |r_b|^2 in
+// one pass (the same per-point formulas as k_residual and k_precond_init; the partials are those that k_reduce would
+// form from R, block by block and in its order, so the norms keep their bits). Bound by memory: a k_reduce of its own
+// read R again. 95^3 x 8, f32: 31.3 us for this kernel and the reduction before, 20.8 us as one. RU points of a thread
+// are loaded together, as many as keep the block's loads in flight.
 template <typename T>
-__global__ void k_residual_precond(T *r, T *w, const T *hx, const T *x, const double *theta, const T *v,
-                                   const double *lam, T diag_t, int nb, long N) {
-    const long i = blockIdx.x * 256L + threadIdx.x;
+__global__ __launch_bounds__(256) void k_residual_precond(T *r, T *w, const T *hx, const T *x, const double *theta,
+                                                          const T *v, const double *lam, T diag_t, long N,
+                                                          double *partials) {
+    constexpr int RU = 4;
+    __shared__ double sh[256];
     const int b = blockIdx.y;
-    if (i >= N) return;
-    const long id = (long)b * N + i;
-    const T rv = (T)((double)hx[id] - theta[b] * (double)x[id]);
-    T d = diag_t + v[i] - (T)lam[b];
-    d = d > T(0.1) ? d : T(0.1);
-    r[id] = rv;
-    w[id] = rv / d;
+    const T *hb = hx + (long)b * N, *xb = x + (long)b * N;
+    T *rb = r + (long)b * N, *wb = w + (long)b * N;
+    const double th = theta[b];
+    const T shift = (T)lam[b];
+    const long stride = (long)RED_BLOCKS * 256;
+    double acc = 0.0;
+    auto point = [&](long p, T hv, T xv, T vv) {
+        const T rv = (T)((double)hv - th * (double)xv);
+        T d = diag_t + vv - shift;
+        d = d > T(0.1) ? d : T(0.1);
+        rb[p] = rv;
+        wb[p] = rv / d;
+        acc += (double)rv * (double)rv;
+    };
+    long p = blockIdx.x * 256L + threadIdx.x;
+    for (; p + (RU - 1) * stride < N; p += RU * stride) {
+        T hv[RU], xv[RU], vv[RU];
+#pragma unroll
+        for (int u = 0; u < RU; u++) {
+            hv[u] = hb[p + u * stride];
+            xv[u] = xb[p + u * stride];
+            vv[u] = v[p + u * stride];
+        }
+#pragma unroll
+        for (int u = 0; u < RU; u++) point(p + u * stride, hv[u], xv[u], vv[u]);
+    }
+    for (; p < N; p += stride) point(p, hb[p], xb[p], v[p]);
+    const double sum = block_sum256(acc, sh);
+    if (threadIdx.x == 0) partials[(long)b * RED_BLOCKS + blockIdx.x] = sum;
 }
 template <typename T>
 void residual_precond(T *r, T *w, const T *hx, const T *x, const double *theta, const T *v, const double *lam,
-                      double diag_t, int nb, long N, hipStream_t s) {
-    if (nb <= 0) return;
-    hipLaunchKernelGGL(k_residual_precond<T>, dim3((unsigned)((N + 255) / 256), nb), dim3(256), 0, s, r, w, hx, x,
-                       theta, v, lam, (T)diag_t, nb, N);
-    LIRA_HIP(hipGetLastError());
+                      double diag_t, int nb, long N, double scale, double *partials, double *norms, hipStream_t s) {
+    for (int b0 = 0; b0 < nb; b0 += MAX_JOBS) {
+        const int cnt = nb - b0 < MAX_JOBS ? nb - b0 : MAX_JOBS;
+        const long off = (long)b0 * N;
+        hipLaunchKernelGGL(k_residual_precond<T>, dim3(RED_BLOCKS, cnt), dim3(256), 0, s, r + off, w + off, hx + off,
+                           x + off, theta + b0, v, lam + b0, (T)diag_t, N, partials);
+        LIRA_HIP(hipGetLastError());
+        KindList kl;
+        for (int j = 0; j < MAX_JOBS; j++) kl.kind[j] = RED_DOT;
+        hipLaunchKernelGGL(k_reduce_finish, dim3(cnt), dim3(256), 0, s, kl, partials, norms + b0, scale);
+        LIRA_HIP(hipGetLastError());
+    }
 }
 
 template <typename T>
@@ -1569,7 +1603,7 @@ void hf_forces(const T *rho, int n, double h, const double *pos, const double *z
     template void reduce_jobs<T>(const RedJobs<T> &, int, double, double *, double *, hipStream_t);                 \
     template void gram<T>(const Cols &, const Cols &, long, double, double *, size_t, double *, hipStream_t);       \
     template void residual_precond<T>(T *, T *, const T *, const T *, const double *, const T *, const double *,     \
-                                      double, int, long, hipStream_t);                                         \
+                                      double, int, long, double, double *, double *, hipStream_t);                    \
     template void lincomb<T>(const Cols &, const double *, int, int, T *, long, hipStream_t, int, T *);                       \
     template void fill<T>(T *, long, double, hipStream_t);                                                           \
     template void axpy<T>(T *, const T *, long, double, hipStream_t);                                                \

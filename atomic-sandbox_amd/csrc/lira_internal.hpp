@@ -88,10 +88,11 @@ size_t gram_partials_needed(int m, int q, long N);
 template <typename T>
 void lincomb(const Cols &S, const double *C, int ldc, int q, T *Y, long N, hipStream_t s, int qsplit = -1,
              T *Y2 = nullptr);
-// R = HX - theta X and W = R / max(diag_t + V - lam, 0.1) for nb bands in one pass
+// R = HX - theta X, W = R / max(diag_t + V - lam, 0.1) and norms[b] = scale |r_b|^2 for nb bands in one pass; partials as
+// in reduce_jobs
 template <typename T>
 void residual_precond(T *r, T *w, const T *hx, const T *x, const double *theta, const T *v, const double *lam,
-                      double diag_t, int nb, long N, hipStream_t s);
+                      double diag_t, int nb, long N, double scale, double *partials, double *norms, hipStream_t s);
 // the padded shape lincomb's coefficients must have: lincomb_rows(m) rows of lincomb_ldc(q) doubles, zero beyond m x q
 int lincomb_rows(int m);
 int lincomb_ldc(int q);

@@ -1357,8 +1357,9 @@ EigenOut Solver<T>::lobpcg(Channel<T> &c, const T *v, int k, double lam, double 
             ra.tol = tol, ra.guess_tol = guess_tol, ra.tail_scale = tol / tail_tol, ra.floor = floor;
             ra.alpha_max = ALPHA_MAX, ra.alpha_fraction = ALPHA_RESIDUAL_FRACTION, ra.drop = RR_DROP;
             auto enqueue = [&](int t) {
+                double *dG = dG_.as<double>();
                 residual_precond<T>(c.R.template as<T>(), c.W.template as<T>(), c.HX.template as<T>(), X(), dth, v,
-                                    dshift, diag_t, k, N_, stream_);
+                                    dshift, diag_t, k, N_, dv_, partials_.as<double>(), dG + (size_t)m * q, stream_);
                 StencilParams jp{n_, na, h_, 1.0, omega, diag_t};
                 for (int sw = 0; sw < 3; sw++) {
                     stencil<T>(ST_JAC, jp, col(c.W, locked), col(c.TMP, locked), v, col(c.R, locked),
@@ -1369,20 +1370,7 @@ EigenOut Solver<T>::lobpcg(Channel<T> &c, const T *v, int k, double lam, double 
                 Cols S{{{X(), k}, {col(c.W, locked), na}, {col(c.P, locked), np}}, 3};
                 Cols U{{{X(), k}, {col(c.W, locked), na}, {col(c.P, locked), np}, {c.R.ptr, k},
                         {col(c.HW, locked), na}, {col(c.HP, locked), np}}, 6};
-                double *dG = dG_.as<double>();
                 gram<T>(S, U, N_, dv_, gpart_.as<double>(), gpart_cap_, dG, stream_);
-                RedJobs<T> jr{};
-                for (int i = 0; i < k; i++) {
-                    jr.a[i % MAX_JOBS] = col(c.R, i);
-                    jr.b[i % MAX_JOBS] = jr.a[i % MAX_JOBS];
-                    jr.kind[i % MAX_JOBS] = RED_DOT;
-                    jr.count = i % MAX_JOBS + 1;
-                    if (jr.count == MAX_JOBS || i == k - 1) {
-                        reduce_jobs<T>(jr, n_, dv_, partials_.as<double>(),
-                                       dG + (size_t)m * q + (i / MAX_JOBS) * MAX_JOBS, stream_);
-                        jr.count = 0;
-                    }
-                }
                 ra.iter = t;
                 ra.record = rr_rec_.as<double>() + (t & 1) * RR_REC_STRIDE;
                 rr_step(ra, stream_);
@@ -1439,8 +1427,8 @@ EigenOut Solver<T>::lobpcg(Channel<T> &c, const T *v, int k, double lam, double 
         }
         const double *dshift = per_column ? dth_cur : dlam;
         // 1. R = HX - theta X for every column (the head's residuals are measured too), W = T R for the moving ones;
-        // three preconditioner sweeps W -> TMP -> W -> TMP (the result in TMP's buffer, which then becomes W); H W and
-        // H P; 2. the Gram B = S^T S and S^T T with S = [X, W, P], T = [R, HW, HP] and ||r_i||^2 for the readback.
+        // and ||r_i||^2 for the readback; three preconditioner sweeps W -> TMP -> W -> TMP (the result in TMP's buffer,
+        // which then becomes W); H W and H P; 2. the Gram B = S^T S and S^T T with S = [X, W, P], T = [R, HW, HP].
         // This device segment is one fixed launch sequence: with graphs on it is captured once per arrangement of
         // its buffers and sizes and replayed (every allocation and tuning it could need done before).
         const int m = k + na + np, q = 2 * m;
@@ -1452,7 +1440,7 @@ EigenOut Solver<T>::lobpcg(Channel<T> &c, const T *v, int k, double lam, double 
         double *dG = dG_.as<double>();
         auto segment = [&] {
             residual_precond<T>(c.R.template as<T>(), W0, c.HX.template as<T>(), X(), dth_cur, v, dshift, diag_t, k, N_,
-                                stream_);
+                                dv_, partials_.as<double>(), dG + (size_t)m * q, stream_);
             StencilParams jp{n_, na, h_, 1.0, omega, diag_t};
             T *const wl = W0 + (long)locked * N_, *const tl = T0 + (long)locked * N_;
             const T *const rl = c.R.template as<T>() + (long)locked * N_;
@@ -1465,18 +1453,6 @@ EigenOut Solver<T>::lobpcg(Channel<T> &c, const T *v, int k, double lam, double 
                     {col(c.HP, locked), np}}, 6};
             if (np == 0) U = Cols{{{X(), k}, {tl, na}, {c.R.ptr, k}, {col(c.HW, locked), na}}, 4};
             gram<T>(S, U, N_, dv_, gpart_.as<double>(), gpart_cap_, dG, stream_);
-            RedJobs<T> jr{};
-            for (int i = 0; i < k; i++) {
-                jr.a[i % MAX_JOBS] = col(c.R, i);
-                jr.b[i % MAX_JOBS] = jr.a[i % MAX_JOBS];
-                jr.kind[i % MAX_JOBS] = RED_DOT;
-                jr.count = i % MAX_JOBS + 1;
-                if (jr.count == MAX_JOBS || i == k - 1) {
-                    reduce_jobs<T>(jr, n_, dv_, partials_.as<double>(), dG + (size_t)m * q + (i / MAX_JOBS) * MAX_JOBS,
-                                   stream_);
-                    jr.count = 0;
-                }
-            }
         };
         const std::vector<uintptr_t> seg_key{
             (uintptr_t)X(), (uintptr_t)W0, (uintptr_t)T0, (uintptr_t)c.R.ptr, (uintptr_t)c.HX.ptr, (uintptr_t)c.HW.ptr,
