@@ -1,7 +1,7 @@
 // gfx950 kernels on the dense n^3 grid: the block stencil H.X, reductions, the tall-skinny Gram S^T U, block
 // linear combinations, density accumulation, LSDA, nuclear potential, orbital guess, DIIS mix and HF forces.
 // All kernels are written for 64-wide wavefronts; reductions are deterministic (fixed partial counts, fixed order).
-#include "lira.h"
+#include "gram_plan.hpp"
 #include "lira_internal.hpp"
 #include "lsda.hpp"
 
@@ -881,47 +881,6 @@ __global__ __launch_bounds__(1024) void k_gram_finish(const double *partials, in
         if (cl < off) sh[cl][o16] += sh[cl + off][o16];
     }
     if (cl == 0 && out < mq) G[out] = sh[0][o16] * scale;
-}
-
-// The tiling of an m x q product: nr x nc tiles of RB x CB 16 x 16 blocks (the blocks split evenly, at most 3 x 6 in f32
-// or where the one tile shares its operands, else 3 x 4: the accumulators and two units of operands fill 256 registers)
-// and the chunks of points. A product of one shared tile takes one workgroup per CU, 16 waves (4 per SIMD, up to 128
-// registers) or 8; several tiles take two 4-wave workgroups per CU, so that the tiles that S^T S's symmetry empties or
-// thins leave room for others. The partials of one product stay within GRAM_PARTIALS doubles (lira_gram_noalloc's fixed
-// array) whenever one chunk's do.
-struct GramPlan {
-    int RB, CB, nr, nc, H, chunks;
-    bool share;
-    long chunk;
-};
-constexpr long GRAM_PARTIALS = (long)(LIRA_NOALLOC_SCRATCH_BYTES / sizeof(double));
-// sym: U's first m columns are S's
-static GramPlan gram_plan(int m, int q, long N, int esize, bool sym) {
-    GramPlan g;
-    const int R = (m + 15) / 16, C = (q + 15) / 16;
-    g.nr = (R + 2) / 3;
-    g.RB = (R + g.nr - 1) / g.nr;
-    g.nr = (R + g.RB - 1) / g.RB;
-    g.share = sym && g.nr == 1 && C <= 6;  // R <= C, for q >= m
-    const int most = esize == 4 || g.share ? 6 : 4;
-    g.nc = (C + most - 1) / most;
-    g.CB = (C + g.nc - 1) / g.nc;
-    g.nc = (C + g.CB - 1) / g.CB;
-    g.H = esize == 4 && g.RB + g.CB <= 5 ? 2 : 1;
-    long want = std::max(1L, (g.share ? 256L : 512L) / (g.nr * g.nc));
-    want = std::max(1L, std::min(want, GRAM_PARTIALS / ((long)m * q)));
-    const long unit = 16 * g.H;
-    g.chunk = ((N + want - 1) / want + unit - 1) / unit * unit;
-    g.chunks = (int)((N + g.chunk - 1) / g.chunk);
-    return g;
-}
-
-size_t gram_partials_needed(int m, int q, long N) {
-    // the precisions, and U beginning with S or not, may split a product differently
-    int chunks = 0;
-    for (int esize : {4, 8})
-        for (bool sym : {false, true}) chunks = std::max(chunks, gram_plan(m, q, N, esize, sym).chunks);
-    return (size_t)chunks * m * q;
 }
 
 static ColPtrs to_ptrs(const Cols &c) {

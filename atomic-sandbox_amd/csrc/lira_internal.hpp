@@ -67,7 +67,8 @@ template <typename T> struct RedJobs {
 template <typename T>
 void reduce_jobs(const RedJobs<T> &jobs, int n, double scale, double *partials, double *out, hipStream_t s);
 
-// G[i * q + j] = scale * sum_p S_i[p] * U_j[p] for i < m, j < q; S columns are segments of band-major blocks.
+// G[i * q + j] = scale * sum_p S_i[p] * U_j[p] for i < m, j < q; S columns are segments of band-major blocks. partials:
+// gram_partials_needed(m, q, N) doubles of scratch (gram_plan.hpp).
 struct Seg {
     const void *base;
     int count;
@@ -81,7 +82,6 @@ struct Cols {
 template <typename T>
 void gram(const Cols &S, const Cols &U, long N, double scale, double *partials, size_t partial_cap, double *G,
           hipStream_t s);
-size_t gram_partials_needed(int m, int q, long N);
 
 // Y_j = sum_i S_i * C[i * q + j] (C f64 on the device, m x q), accumulated in f64. Outputs j < qsplit go to
 // Y + j N, the others to Y2 + (j - qsplit) N.

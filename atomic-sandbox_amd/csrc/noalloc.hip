@@ -7,6 +7,7 @@
 #include <mutex>
 
 #include "lira.h"
+#include "gram_plan.hpp"
 #include "lira_internal.hpp"
 
 namespace {

@@ -21,6 +21,7 @@
 #include <type_traits>
 
 #include "lira.h"
+#include "gram_plan.hpp"
 #include "lira_internal.hpp"
 #include "provider_policy.hpp"
 
@@ -815,8 +816,9 @@ template <typename T> class Solver final : public SolverIface {
     void alloc_field(DevBuf &b, int count = 1) {
         if (b.bytes < (size_t)N_ * count * sizeof(T)) b.alloc((size_t)N_ * count * sizeof(T));
     }
+    // for every Gram of at most m x q columns
     void ensure_gram(int m, int q) {
-        const size_t need = gram_partials_needed(m, q, N_);
+        const size_t need = gram_partials_bound(m, q, N_);
         if (need > gpart_cap_) {
             gpart_.alloc(need * sizeof(double));
             gpart_cap_ = need;
@@ -1295,7 +1297,7 @@ EigenOut Solver<T>::lobpcg(Channel<T> &c, const T *v, int k, double lam, double 
     }
     auto X = [&]() { return c.X.template as<T>(); };
     auto col = [&](DevBuf &b, int i) { return b.template as<T>() + (long)i * N_; };
-    ensure_gram(3 * k, 6 * k);
+    ensure_gram(3 * k, 6 * k);  // the guess's k x 2k product and every step's
     // the guess: B = X^T X and the Rayleigh quotients theta_i = <x_i, H x_i> / <x_i, x_i>
     std::vector<double> theta(k);
     for (int round = 0;; round++) {
