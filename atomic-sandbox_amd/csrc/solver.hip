@@ -767,6 +767,7 @@ template <typename T> class Solver final : public SolverIface {
     void nl_apply_block(const T *x, T *out, int nb, const T *x2 = nullptr, T *out2 = nullptr, int nb2 = 0);
     void nl_projections(const T *x, int nb);
     long nl_max_pts() const;
+    void nl_launch_key(std::vector<uintptr_t> &key) const;
     void ensure_nl(int nb);  // the projections' buffers for nb bands
     std::vector<double> nl_energy_terms(Channel<T> &c, bool fd);
 
@@ -1456,12 +1457,13 @@ EigenOut Solver<T>::lobpcg(Channel<T> &c, const T *v, int k, double lam, double 
             if (np == 0) U = Cols{{{X(), k}, {tl, na}, {c.R.ptr, k}, {col(c.HW, locked), na}}, 4};
             gram<T>(S, U, N_, dv_, gpart_.as<double>(), gpart_cap_, dG, stream_);
         };
-        const std::vector<uintptr_t> seg_key{
+        std::vector<uintptr_t> seg_key{
             (uintptr_t)X(), (uintptr_t)W0, (uintptr_t)T0, (uintptr_t)c.R.ptr, (uintptr_t)c.HX.ptr, (uintptr_t)c.HW.ptr,
             (uintptr_t)c.HP.ptr, (uintptr_t)c.P.ptr, (uintptr_t)v, (uintptr_t)dth_cur, (uintptr_t)dshift, (uintptr_t)dG,
             (uintptr_t)gpart_.ptr, (uintptr_t)partials_.ptr, (uintptr_t)nl_C_.ptr, (uintptr_t)nl_P_.ptr,
             (uintptr_t)beta_.ptr, (uintptr_t)k, (uintptr_t)na, (uintptr_t)np,
             (uintptr_t)locked, (uintptr_t)vj, (uintptr_t)nl_rows_, (uintptr_t)ionic_version_};
+        nl_launch_key(seg_key);
         run_graph(lobpcg_graph_[W0 < T0 ? 0 : 1], seg_key, segment);
         std::swap(c.W, c.TMP);  // the sweeps' result sits in TMP's buffer
         const double *g = readback(dG, (size_t)m * q + k);
@@ -1978,6 +1980,14 @@ template <typename T> long Solver<T>::nl_max_pts() const {
     long m = 0;
     for (const NlIon &ion : nl_h_) m = std::max(m, ion.pts);
     return m;
+}
+
+// Appends what the launches of nl_apply_block hold of the geometry: the box sizes and ion count that fix their chunks, the
+// colours, and the tables that a geometry may have moved. A graph that was captured with other ones is not replayed.
+template <typename T> void Solver<T>::nl_launch_key(std::vector<uintptr_t> &key) const {
+    key.insert(key.end(), {(uintptr_t)nl_max_pts(), (uintptr_t)nl_h_.size(), (uintptr_t)nl_ions_.ptr,
+                           (uintptr_t)nl_members_.ptr, (uintptr_t)nl_erow_.ptr});
+    for (const Colour &c : colours_) key.insert(key.end(), {(uintptr_t)c.off, (uintptr_t)c.count});
 }
 
 template <typename T> void Solver<T>::nl_projections(const T *x, int nb) {
