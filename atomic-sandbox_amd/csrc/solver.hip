@@ -22,6 +22,7 @@
 
 #include "lira.h"
 #include "gram_plan.hpp"
+#include "host_stage.hpp"
 #include "lira_internal.hpp"
 #include "provider_policy.hpp"
 
@@ -453,34 +454,25 @@ class HostStage {
     char *slots_[WORKERS][SLOTS] = {};
     hipEvent_t ev_[WORKERS][SLOTS] = {};
 
-    // chunks first, first + step, ... of one worker; every copy that it queued has completed when it returns
-    hipError_t work(int w, int step, char *dev, char *host, size_t bytes, bool to_device, hipStream_t s) {
-        const size_t chunks = (bytes + SLOT - 1) / SLOT;
-        hipError_t err = hipSuccess;
-        size_t queued[SLOTS];  // the chunk in flight in each slot, or chunks
-        for (size_t &q : queued) q = chunks;
-        auto len = [&](size_t c) { return std::min(SLOT, bytes - c * SLOT); };
-        auto finish = [&](int j) {  // wait for the slot's copy; on the way to the host its data moves on
-            if (queued[j] == chunks) return;
-            const hipError_t e = hipEventSynchronize(ev_[w][j]);
-            if (err == hipSuccess) err = e;
-            if (!to_device && err == hipSuccess) std::memcpy(host + queued[j] * SLOT, slots_[w][j], len(queued[j]));
-            queued[j] = chunks;
-        };
-        int j = 0;
-        for (size_t c = (size_t)w; c < chunks && err == hipSuccess; c += (size_t)step, j = (j + 1) % SLOTS) {
-            finish(j);
-            if (err != hipSuccess) break;
-            if (to_device) std::memcpy(slots_[w][j], host + c * SLOT, len(c));
-            hipError_t e = to_device
-                               ? hipMemcpyAsync(dev + c * SLOT, slots_[w][j], len(c), hipMemcpyHostToDevice, s)
-                               : hipMemcpyAsync(slots_[w][j], dev + c * SLOT, len(c), hipMemcpyDeviceToHost, s);
-            if (e == hipSuccess) e = hipEventRecord(ev_[w][j], s);
-            if (e != hipSuccess) err = e;
-            else queued[j] = c;
+    // one worker's slots, for stage_chunks
+    struct Link {
+        char *const *slots;
+        const hipEvent_t *ev;
+        char *dev;
+        bool to_device;
+        hipStream_t s;
+        char *slot(int j) const { return slots[j]; }
+        hipError_t copy(int j, size_t off, size_t len) const {
+            return to_device ? hipMemcpyAsync(dev + off, slots[j], len, hipMemcpyHostToDevice, s)
+                             : hipMemcpyAsync(slots[j], dev + off, len, hipMemcpyDeviceToHost, s);
         }
-        for (int k = 0; k < SLOTS; k++, j = (j + 1) % SLOTS) finish(j);
-        return err;
+        hipError_t record(int j) const { return hipEventRecord(ev[j], s); }
+        hipError_t wait(int j) const { return hipEventSynchronize(ev[j]); }
+        hipError_t drain() const { return hipStreamSynchronize(s); }
+    };
+    hipError_t work(int w, int step, char *dev, char *host, size_t bytes, bool to_device, hipStream_t s) {
+        const Link link{slots_[w], ev_[w], dev, to_device, s};
+        return stage_chunks<SLOTS, hipError_t>(link, host, bytes, SLOT, to_device, (size_t)w, (size_t)step);
     }
 
     void copy(void *dev, void *host, size_t bytes, bool to_device, hipStream_t s) {
