@@ -704,20 +704,72 @@ __device__ inline const void *col_base(const ColPtrs &c, int col, long N, int es
 // in every precision mode.
 //
 // The operands go from memory to the matrix cores without LDS. The order in which points enter the sum is free, so a lane
-// loads four consecutive points of its column (16 bytes in f32, 32 in f64: column l % 16 of a 16-column block, points
-// 4 (l / 16) .. + 3 of a 16-point stage) and feeds one of them to each of four MFMAs; A and B share that layout, so a
+// loads 16 bytes of consecutive points and feeds one of them to each MFMA (GramLoad); A and B share that layout, so a
 // column block that is both (S^T S, SHARE) is loaded once. A wave holds RB x CB output blocks: per 16 points RB + CB
-// loads and conversions of 4 values against 4 RB CB MFMAs (64 cycles each), one unit of 16 H points in flight while the
+// blocks loaded and converted against 4 RB CB MFMAs (64 cycles each), one unit of points in flight while the
 // previous one is multiplied. The waves of a workgroup take interleaved units of its chunk of points and their blocks
 // are summed in wave order; the workgroups that share a chunk run next to each other on one XCD, so its columns
 // come from that L2. (Before, each wave staged its columns through LDS as f64 with a pointer lookup per load: 24 x 48
 // columns on 95^3 f32 60 us, 138 x 276 on 160^3 11 ms.)
 typedef double lira_d4 __attribute__((ext_vector_type(4)));
 
-// four consecutive values at any element alignment, in the global address space
-template <typename T> struct Quad {
-    typedef T type __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+// What a lane loads of one 16-column block, and operand j of its unit: a value of column l % 16, at the same point in every
+// block.
+// QUAD: four points (16 bytes in f32, 32 in f64) of column l % 16, 4 (l / 16) .. + 3 of 16, H times. One instruction takes
+// 64 bytes of each of 16 columns.
+template <typename T, int H, int LOADS> struct GramLoad;
+template <typename T, int H> struct GramLoad<T, H, GRAM_QUAD> {
+    typedef T Q __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+    static constexpr int COLS = 1, P = 4 * H;
+    Q v[H];
+    __device__ static int column(int lane, int) { return lane & 15; }
+    __device__ static int point(int lane, int j) { return 16 * (j / 4) + 4 * (lane >> 4) + j % 4; }
+    __device__ static int source(int) { return 0; }
+    __device__ void load(const T *const *c, long p, int lane) {
+#pragma unroll
+        for (int h = 0; h < H; h++) v[h] = *(const __attribute__((address_space(1))) Q *)(c[0] + p + point(lane, 4 * h));
+    }
+    __device__ void set(int j, T x) { v[j / 4][j % 4] = x; }
+    __device__ double operand(int j) const { return (double)v[j / 4][j % 4]; }
 };
+// PAIR: 16 bytes of columns l % 8 and l % 8 + 8, at piece l / 8 of 128 bytes, H times. One instruction takes 128 bytes of
+// each of 8 columns, so the columns cost half as many requests and address translations; lanes l and l ^ 8 of a
+// row of 16 then exchange the halves that are not their column's (a move each, no select: the other banks keep theirs).
+// f64, kernels of both loads: 24 x 48 on 95^3 86 -> 75 us, on 128^3 222 -> 171 (173 with the LDS kernel before), on 192^3
+// 733 -> 523 (539); 32 x 64 on 128^3 318 -> 223. Where the columns stay in the 256 MiB cache it gains nothing. With two
+// loads of a column in flight (PAIR2) 32 x 64 on 192^3 755 -> 700 us, on 256^3 2303 -> 1641, but on 95^3 91 -> 97.
+// f32, where both take 64 or 128 bytes of a column: it gains where a stride of a multiple of 8 MiB puts all columns on the
+// same channels (32 x 64 on 128^3 176 -> 139 us, on 256^3 1611 -> 1000) and costs elsewhere (on 95^3 57 -> 62).
+template <typename T, int H> struct GramLoad<T, H, GRAM_PAIR> {
+    static constexpr int COLS = 2, VX = 16 / (int)sizeof(T), P = 2 * VX * H;
+    typedef T V __attribute__((ext_vector_type(VX), aligned(sizeof(T))));
+    V v[2 * H];  // per depth the first column's points, then the second's
+    __device__ static int column(int lane, int i) { return (lane & 7) + 8 * i; }
+    __device__ static int point(int lane, int j) { return 8 * VX * (j / (2 * VX)) + VX * (lane >> 3) + j % VX; }
+    __device__ static int source(int j) { return j / VX % 2; }
+    __device__ void load(const T *const *c, long p, int lane) {
+#pragma unroll
+        for (int i = 0; i < 2 * H; i++)
+            v[i] = *(const __attribute__((address_space(1))) V *)(c[i % 2] + p + point(lane, VX * i));
+    }
+    __device__ void set(int j, T x) { v[j / VX][j % VX] = x; }
+    // lanes of BANKS (four lanes each) take `from` of the lane eight over, the others `keep`
+    template <int BANKS> __device__ static int cross(int keep, int from) {
+        return __builtin_amdgcn_update_dpp(keep, from, 0x128, 0xf, BANKS, false);  // row_ror:8
+    }
+    template <int BANKS> __device__ static float cross(float keep, float from) {
+        return __builtin_bit_cast(float, cross<BANKS>(__builtin_bit_cast(int, keep), __builtin_bit_cast(int, from)));
+    }
+    template <int BANKS> __device__ static double cross(double keep, double from) {
+        const int2 k = __builtin_bit_cast(int2, keep), f = __builtin_bit_cast(int2, from);
+        return __builtin_bit_cast(double, int2{cross<BANKS>(k.x, f.x), cross<BANKS>(k.y, f.y)});
+    }
+    __device__ double operand(int j) const {
+        const int i = j / VX, e = j % VX;
+        return (double)(i % 2 == 0 ? cross<0xc>(T(v[i][e]), T(v[i + 1][e])) : cross<0x3>(T(v[i][e]), T(v[i - 1][e])));
+    }
+};
+template <typename T, int H> struct GramLoad<T, H, GRAM_PAIR2> : GramLoad<T, H, GRAM_PAIR> {};
 
 // With sym (U's first m columns are S's), the 16 x 16 blocks of S^T S strictly below its diagonal are skipped
 // (gram_mirrored): k_gram_finish reads their values from the transposed block, the same sum of the same exact products.
@@ -726,17 +778,14 @@ __host__ __device__ inline bool gram_mirrored(int sym, int m, int i, int j) {
     return sym && cb < rb && 16 * (cb + 1) <= m;
 }
 
-// W waves of a workgroup
-__host__ __device__ constexpr int gram_waves(int RB, int CB, bool SHARE) {
-    return !SHARE ? 4 : RB * CB <= 6 && CB <= 3 ? 16 : 8;
-}
-template <typename T, int RB, int CB, bool SHARE, int H>
-__global__ __launch_bounds__(64 * gram_waves(RB, CB, SHARE), gram_waves(RB, CB, SHARE) == 16 ? 4 : 2) void k_gram(ColPtrs S, ColPtrs U, int m, int q, long N, long chunk, int chunks, int nc,
-                                              int nsub, double *partials, int sym) {
-    typedef typename Quad<T>::type Q;
-    constexpr int UP = 16 * H;           // points of a wave's unit
-    constexpr int NB = SHARE ? CB : RB + CB;  // column blocks loaded
-    constexpr int W = gram_waves(RB, CB, SHARE);
+template <typename T, int RB, int CB, bool SHARE, int LOADS>
+__global__ __launch_bounds__(64 * gram_waves(RB, CB, SHARE), gram_waves(RB, CB, SHARE) == 16 ? 4 : 2) void k_gram(
+    ColPtrs S, ColPtrs U, int m, int q, long N, long chunk, int chunks, int nc, int nsub, double *partials, int sym) {
+    constexpr int H = gram_depth(RB, CB, sizeof(T), LOADS), W = gram_waves(RB, CB, SHARE);
+    typedef GramLoad<T, H, LOADS> Load;
+    constexpr int UP = gram_unit(H, sizeof(T), LOADS);  // points of a wave's unit
+    static_assert(UP == 4 * Load::P, "four lanes of a column hold a unit");
+    constexpr int NB = gram_loaded(RB, CB, SHARE);  // column blocks loaded
     __shared__ double red[W][256];
     const int total = chunks * nsub, per = (total + 7) / 8;
     const int L = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
@@ -754,14 +803,19 @@ __global__ __launch_bounds__(64 * gram_waves(RB, CB, SHARE), gram_waves(RB, CB, 
             if (i0 + 16 * a < m && j0 + 16 * b < q && !gram_mirrored(sym, m, i0 + 16 * a, j0 + 16 * b))
                 live |= 1u << (a * CB + b);
     if (live == 0) return;
-    // this lane's column of each block; past the last column it reads that one (its outputs are not stored)
-    const T *col[NB];
+    // this lane's columns of each block; past the last column it reads that one (its outputs are not stored)
+    const T *col[NB][Load::COLS];
 #pragma unroll
-    for (int b = 0; b < CB; b++) col[b] = static_cast<const T *>(col_base(U, min(j0 + 16 * b + c16, q - 1), N, sizeof(T)));
-    if constexpr (!SHARE) {
+    for (int i = 0; i < Load::COLS; i++) {
+        const int c = Load::column(lane, i);
 #pragma unroll
-        for (int a = 0; a < RB; a++)
-            col[CB + a] = static_cast<const T *>(col_base(S, min(i0 + 16 * a + c16, m - 1), N, sizeof(T)));
+        for (int b = 0; b < CB; b++)
+            col[b][i] = static_cast<const T *>(col_base(U, min(j0 + 16 * b + c, q - 1), N, sizeof(T)));
+        if constexpr (!SHARE) {
+#pragma unroll
+            for (int a = 0; a < RB; a++)
+                col[CB + a][i] = static_cast<const T *>(col_base(S, min(i0 + 16 * a + c, m - 1), N, sizeof(T)));
+        }
     }
     lira_d4 acc[RB][CB];
 #pragma unroll
@@ -772,34 +826,30 @@ __global__ __launch_bounds__(64 * gram_waves(RB, CB, SHARE), gram_waves(RB, CB, 
     const long units = p_end > p_begin ? (p_end - p_begin) / UP : 0;  // whole units; the rest is the last chunk's tail
     // the products of one unit; ALL: every block of the tile is live. (A SHARE tile is the whole product, so its dead
     // blocks are those with b < a, known here.)
-    auto multiply = [&](const Q(&v)[H][NB], auto all) {
+    auto multiply = [&](const Load(&v)[NB], auto all) {
 #pragma unroll
-        for (int h = 0; h < H; h++)
+        for (int j = 0; j < Load::P; j++) {
+            double x[NB];
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                double x[NB];
+            for (int b = 0; b < NB; b++) x[b] = v[b].operand(j);
 #pragma unroll
-                for (int b = 0; b < NB; b++) x[b] = (double)v[h][b][j];
+            for (int a = 0; a < RB; a++)
 #pragma unroll
-                for (int a = 0; a < RB; a++)
-#pragma unroll
-                    for (int b = SHARE ? a : 0; b < CB; b++)
-                        if (SHARE || decltype(all)::value || (live >> (a * CB + b)) & 1u)
-                            acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[SHARE ? a : CB + a], x[b], acc[a][b], 0, 0, 0);
-            }
+                for (int b = SHARE ? a : 0; b < CB; b++)
+                    if (SHARE || decltype(all)::value || (live >> (a * CB + b)) & 1u)
+                        acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[SHARE ? a : CB + a], x[b], acc[a][b], 0, 0, 0);
+        }
     };
     auto run = [&](auto all) {
         if (units > 0) {
             // every load is issued unconditionally (a load under a branch would be waited for at the join): past the
             // wave's last unit it reads the chunk's last unit again, which is not multiplied
-            auto fetch = [&](long u, Q(&v)[H][NB]) {
-                const long p = p_begin + min(u, units - 1) * UP + 4 * k4;
+            auto fetch = [&](long u, Load(&v)[NB]) {
+                const long p = p_begin + min(u, units - 1) * UP;
 #pragma unroll
-                for (int b = 0; b < NB; b++)
-#pragma unroll
-                    for (int h = 0; h < H; h++) v[h][b] = *(const __attribute__((address_space(1))) Q *)(col[b] + p + 16 * h);
+                for (int b = 0; b < NB; b++) v[b].load(col[b], p, lane);
             };
-            Q va[H][NB], vb[H][NB];
+            Load va[NB], vb[NB];
             long u = wave;
             fetch(u, va);
             for (; u + W < units; u += 2 * W) {
@@ -812,16 +862,14 @@ __global__ __launch_bounds__(64 * gram_waves(RB, CB, SHARE), gram_waves(RB, CB, 
         }
         const long pt = p_begin + units * UP;
         if (pt < p_end && wave == (int)(units % W)) {  // the tail, fewer than UP points: guarded loads
-            Q v[H][NB];
+            Load v[NB];
 #pragma unroll
             for (int b = 0; b < NB; b++)
 #pragma unroll
-                for (int h = 0; h < H; h++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const long p = pt + 16 * h + 4 * k4 + j;
-                        v[h][b][j] = p < p_end ? gload(col[b] + p) : T(0);
-                    }
+                for (int j = 0; j < Load::P; j++) {
+                    const long p = pt + Load::point(lane, j);
+                    v[b].set(j, p < p_end ? gload(col[b][Load::source(j)] + p) : T(0));
+                }
             multiply(v, all);
         }
     };
@@ -900,10 +948,18 @@ template <typename T, int RB, int CB, bool SHARE>
 static void launch_gram(const GramPlan &g, const ColPtrs &sp, const ColPtrs &up, int m, int q, long N, double *partials,
                         int sym, hipStream_t s) {
     const int total = g.chunks * g.nr * g.nc;
-    const dim3 grid((unsigned)(8 * ((total + 7) / 8)));
-    constexpr bool TWO = sizeof(T) == 4 && RB + CB <= 5;
-    hipLaunchKernelGGL((k_gram<T, RB, CB, SHARE, TWO ? 2 : 1>), grid, dim3(64 * gram_waves(RB, CB, SHARE)), 0, s, sp, up, m, q, N, g.chunk, g.chunks,
-                       g.nc, g.nr * g.nc, partials, sym);
+    const dim3 grid((unsigned)(8 * ((total + 7) / 8))), block(64 * gram_waves(RB, CB, SHARE));
+    auto go = [&](auto loads) {
+        constexpr int L = decltype(loads)::value;
+        if constexpr (gram_has(RB, CB, SHARE, sizeof(T), L)) {
+            if (g.loads == L)
+                hipLaunchKernelGGL((k_gram<T, RB, CB, SHARE, L>), grid, block, 0, s, sp, up, m, q, N, g.chunk, g.chunks, g.nc,
+                                   g.nr * g.nc, partials, sym);
+        }
+    };
+    go(std::integral_constant<int, GRAM_QUAD>{});
+    go(std::integral_constant<int, GRAM_PAIR>{});
+    go(std::integral_constant<int, GRAM_PAIR2>{});
 }
 
 template <typename T>

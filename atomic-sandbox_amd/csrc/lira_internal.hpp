@@ -68,7 +68,7 @@ template <typename T>
 void reduce_jobs(const RedJobs<T> &jobs, int n, double scale, double *partials, double *out, hipStream_t s);
 
 // G[i * q + j] = scale * sum_p S_i[p] * U_j[p] for i < m, j < q; S columns are segments of band-major blocks. partials:
-// gram_partials_needed(m, q, N) doubles of scratch (gram_plan.hpp).
+// gram_partials doubles of scratch (gram_plan.hpp).
 struct Seg {
     const void *base;
     int count;

@@ -48,7 +48,7 @@ extern "C" lira_status lira_gram_noalloc(int dtype, int n, double h, int m, cons
         return LIRA_INVALID;
     const long N = (long)n * n * n;
     // the partials of this shape must fit the fixed array (checked before anything touches the device)
-    if (lira::gram_partials_needed(m, q, N) > SCRATCH_DOUBLES) return LIRA_INVALID;
+    if (lira::gram_partials(m, q, N, dtype, s_block == u_block && q >= m) > SCRATCH_DOUBLES) return LIRA_INVALID;
     lira_status st = LIRA_OK;
     double *part = scratch_on_current_device(&st);
     if (st != LIRA_OK) return st;

@@ -3901,7 +3901,8 @@ lira_status lira_gram(int dtype, int n, double h, int m, const void *s_block, in
     if ((dtype != 4 && dtype != 8) || n < 1 || m < 1 || q < 1 || !s_block || !u_block || !g) return LIRA_INVALID;
     return guarded(nullptr, [&] {
         const long N = (long)n * n * n;
-        const size_t need = gram_partials_needed(m, q, N);
+        // sized by the plan that gram takes: allocations of megabytes are what a call on a small grid spends its time on
+        const size_t need = gram_partials(m, q, N, dtype, s_block == u_block && q >= m);
         DevBuf part(need * sizeof(double)), dg((size_t)m * q * sizeof(double));
         Cols S{{{s_block, m}}, 1}, U{{{u_block, q}}, 1};
         if (dtype == 4) gram<float>(S, U, N, h * h * h, part.as<double>(), need, dg.as<double>(), as_stream(stream));

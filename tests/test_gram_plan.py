@@ -24,15 +24,14 @@ int main() {
                 for (int m = 1; m <= 384; m++)
                     for (int q : {1, m / 2 + 1, m, 2 * m}) {
                         const long N = (long)n * n * n;
-                        const size_t need = (size_t)lira::gram_plan(m, q, N, esize, sym && q >= m).chunks * m * q;
-                        if (need > lira::gram_partials_needed(m, q, N)) bad++;
+                        const size_t need = lira::gram_partials(m, q, N, esize, sym && q >= m);
                         if (need > lira::gram_partials_bound(m, q, N)) bad++;
                         // growing in both, so a buffer for (m, q) serves every product within it
                         if (lira::gram_partials_bound(m, q, N) > lira::gram_partials_bound(m + 1, q, N)) bad++;
                         if (lira::gram_partials_bound(m, q, N) > lira::gram_partials_bound(m, q + 1, N)) bad++;
                         if (q == 2 * m && m <= 128) {
                             if (need > lira::gram_partials_bound(3 * m, 6 * m, N)) bad++;
-                            if (need > lira::gram_partials_needed(3 * m, 6 * m, N)) inverted++;
+                            if (need > lira::gram_partials(3 * m, 6 * m, N, esize, sym)) inverted++;
                         }
                     }
     std::printf("%ld refused, %ld need more than three times their columns\n", bad, inverted);
