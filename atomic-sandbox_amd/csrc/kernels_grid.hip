@@ -3,7 +3,6 @@
 // All kernels are written for 64-wide wavefronts; reductions are deterministic (fixed partial counts, fixed order).
 #include "gram_plan.hpp"
 #include "lira_internal.hpp"
-#include "lsda.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -96,9 +95,9 @@ struct StWork {
     int tile_x, tile_y, band, zchunk;
     bool valid;
 };
-// order 0: tiles fastest, then z chunks, then bands; 1: bands fastest; G >= 2: bands in groups of G fastest, then
-// tiles, then z chunks, then groups — the G bands of a tile share V in L2 while neighbouring tiles (the halos) run
-// side by side. Bands padded to a multiple of G are skipped.
+// order 0: tiles fastest, then z chunks, then bands; G >= 2: bands in groups of G fastest, then tiles, then z chunks,
+// then groups: the G bands of a tile share V in L2 while neighbouring tiles (the halos) run side by side. Bands padded
+// to a multiple of G are skipped.
 __device__ __forceinline__ StWork st_decode(int ntx, int nty, int nzc, int nb, int order) {
     const int tiles = ntx * nty;
     const int nbp = order >= 2 ? ((nb + order - 1) / order) * order : nb;
@@ -114,11 +113,6 @@ __device__ __forceinline__ StWork st_decode(int ntx, int nty, int nzc, int nb, i
         rest = L / tiles;
         w.zchunk = rest % nzc;
         w.band = rest / nzc;
-    } else if (order == 1) {
-        w.band = L % nb;
-        rest = L / nb;
-        tile = rest % tiles;
-        w.zchunk = rest / tiles;
     } else {
         const int gi = L % order;
         rest = L / order;
@@ -432,7 +426,7 @@ __global__ __launch_bounds__(TXL *TYL) __attribute__((amdgpu_waves_per_eu(3))) v
 struct StVariant {
     int tx;     // tile width in points
     int zc;     // planes per chunk; 0: whole columns, -1: chunks that load the CUs evenly
-    int order;  // XCD work order: 0 tiles fastest, 1 bands fastest, G >= 2 bands in groups of G fastest
+    int order;  // XCD work order: 0 tiles fastest, G >= 2 bands in groups of G fastest
     const char *name;
 };
 static const StVariant ST_VARIANTS[] = {
@@ -1106,7 +1100,7 @@ template <typename T> void residual(T *r, const T *hx, const T *x, const double 
 }
 
 // R = HX - theta X, the preconditioner's first pass W = R / max(diag_t + V - lam, 0.1) and the partial sums of |r_b|^2 in
-// one pass (the same per-point formulas as k_residual and k_precond_init; the partials are those that k_reduce would
+// one pass (k_residual's formula; the partials are those that k_reduce would
 // form from R, block by block and in its order, so the norms keep their bits). Bound by memory: a k_reduce of its own
 // read R again. 95^3 x 8, f32: 31.3 us for this kernel and the reduction before, 20.8 us as one. RU points of a thread
 // are loaded together, as many as keep the block's loads in flight.
@@ -1161,23 +1155,6 @@ void residual_precond(T *r, T *w, const T *hx, const T *x, const double *theta, 
         hipLaunchKernelGGL(k_reduce_finish, dim3(cnt), dim3(256), 0, s, kl, partials, norms + b0, scale);
         LIRA_HIP(hipGetLastError());
     }
-}
-
-template <typename T>
-__global__ void k_precond_init(T *w, const T *r, const T *v, const double *lam, T diag_t, int nb, long N) {
-    const long i = blockIdx.x * 256L + threadIdx.x;
-    const int b = blockIdx.y;
-    if (i >= N) return;
-    T d = diag_t + v[i] - (T)lam[b];
-    d = d > T(0.1) ? d : T(0.1);
-    w[(long)b * N + i] = r[(long)b * N + i] / d;
-}
-template <typename T>
-void precond_init(T *w, const T *r, const T *v, const double *lam, double diag_t, int nb, long N, hipStream_t s) {
-    if (nb <= 0) return;
-    hipLaunchKernelGGL(k_precond_init<T>, dim3((unsigned)((N + 255) / 256), nb), dim3(256), 0, s, w, r, v, lam,
-                       (T)diag_t, nb, N);
-    LIRA_HIP(hipGetLastError());
 }
 
 template <typename T> __global__ void k_density(T *rho, const T *psi, const double *f, int nb, long N) {
@@ -1623,7 +1600,6 @@ void hf_forces(const T *rho, int n, double h, const double *pos, const double *z
     template void fill<T>(T *, long, double, hipStream_t);                                                           \
     template void axpy<T>(T *, const T *, long, double, hipStream_t);                                                \
     template void residual<T>(T *, const T *, const T *, const double *, int, long, hipStream_t);                    \
-    template void precond_init<T>(T *, const T *, const T *, const double *, double, int, long, hipStream_t);        \
     template void density<T>(T *, const T *, const double *, int, long, hipStream_t);                                \
     template void sum3<T>(T *, const T *, const T *, const T *, long, hipStream_t);                                  \
     template void add2<T>(T *, const T *, const T *, long, hipStream_t);                                             \

@@ -131,9 +131,6 @@ template <typename T> void fill(T *y, long count, double a, hipStream_t s);
 template <typename T> void axpy(T *y, const T *x, long count, double a, hipStream_t s);  // y += a x
 // r_b = hx_b - theta_b x_b, theta on the device (f64)
 template <typename T> void residual(T *r, const T *hx, const T *x, const double *theta, int nb, long N, hipStream_t s);
-// w_b = r_b / max(diag_t + v - lam_b, 0.1)
-template <typename T>
-void precond_init(T *w, const T *r, const T *v, const double *lam, double diag_t, int nb, long N, hipStream_t s);
 // rho = sum_b f_b psi_b^2 (f on the device, f64)
 template <typename T> void density(T *rho, const T *psi, const double *f, int nb, long N, hipStream_t s);
 // v_sigma = vnuc + vh + vxc_sigma

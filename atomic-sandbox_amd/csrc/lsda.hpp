@@ -1,13 +1,13 @@
 // LSDA exchange-correlation at one point: Dirac exchange + PW92 correlation with the spin interpolation, f64
-// (qm/src/xc.rs:120-210). Shared by the XC kernel and the host free-atom solver.
+// (qm/src/xc.rs:120-210), for the host's free-atom and pseudopotential solvers. The XC kernel has the same formulas in
+// its own forms of the roots, logarithms and quotients (lsda_point in kernels_grid.hip): a change of one is a change of
+// both.
 #pragma once
-#include <hip/hip_runtime.h>
 #include <cmath>
 
 namespace lira {
 
-__host__ __device__ inline void pw92_g(double rs, double a, double a1, double b1, double b2, double b3, double b4, double &g,
-                              double &dg) {
+inline void pw92_g(double rs, double a, double a1, double b1, double b2, double b3, double b4, double &g, double &dg) {
     const double srs = sqrt(rs);
     const double q0 = -2.0 * a * (1.0 + a1 * rs);
     const double q1 = 2.0 * a * (b1 * srs + b2 * rs + b3 * rs * srs + b4 * rs * rs);
@@ -17,7 +17,7 @@ __host__ __device__ inline void pw92_g(double rs, double a, double a1, double b1
     dg = -2.0 * a * a1 * ln - q0 * q1p / (q1 * q1 + q1);
 }
 
-__host__ __device__ inline void exc_point(double nu, double nd, double &e, double &vu, double &vd) {
+inline void exc_point(double nu, double nd, double &e, double &vu, double &vd) {
     nu = nu > 0.0 ? nu : 0.0;
     nd = nd > 0.0 ? nd : 0.0;
     const double n = nu + nd;
