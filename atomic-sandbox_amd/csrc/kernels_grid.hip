@@ -106,22 +106,14 @@ __device__ __forceinline__ StWork st_decode(int ntx, int nty, int nzc, int nb, i
     const int lin = blockIdx.x;
     const int L = (lin & 7) * per + (lin >> 3);
     StWork w;
-    w.valid = L < total;
-    int tile, rest;
-    if (order == 0) {
-        tile = L % tiles;
-        rest = L / tiles;
-        w.zchunk = rest % nzc;
-        w.band = rest / nzc;
-    } else {
-        const int gi = L % order;
-        rest = L / order;
-        tile = rest % tiles;
-        rest = rest / tiles;
-        w.zchunk = rest % nzc;
-        w.band = (rest / nzc) * order + gi;
-        w.valid = w.valid && w.band < nb;
-    }
+    const int group = order >= 2 ? order : 1;
+    const int gi = L % group;
+    int rest = L / group;
+    const int tile = rest % tiles;
+    rest /= tiles;
+    w.zchunk = rest % nzc;
+    w.band = (rest / nzc) * group + gi;
+    w.valid = L < total && w.band < nb;
     w.tile_x = tile % ntx;
     w.tile_y = tile / ntx;
     return w;
