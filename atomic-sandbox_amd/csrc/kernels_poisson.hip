@@ -602,7 +602,7 @@ template <typename T> __global__ __launch_bounds__(256) void k_mg_prolong_cells(
 // a zero border (one column after each row, one row after each plane, a plane at either end), so no neighbour read is a
 // branch; a column's diagonal takes three values (first, inner and last plane). Levels of at most 8^2 columns run on the
 // first wave alone, without block barriers. What bounds it is the chain of some 60 LDS latencies and barriers: f64 from
-// 12^3 36.5 -> 14.4 us, f32 from 16^3 50.7 -> 16.1 us (the levels as loops of 1024 threads over all points, every index
+// 12^3 36.5 -> 13.5 us, f32 from 16^3 50.7 -> 15.0 us (the levels as loops of 1024 threads over all points, every index
 // divided out and every neighbour behind a branch, before). Entering at 24^3 instead (a 576-thread workgroup, 36 us)
 // saved seven launches and took as long as they do (a Hartree solve on 95^3: 3.67 ms against 3.54).
 // one level's LDS array: border, then plane k, row j, point i at (1 + k) (NMAX + 1)^2 + j (NMAX + 1) + i + 1
@@ -619,10 +619,10 @@ static constexpr int mgc_threads(int nmax) { return (nmax * nmax + 63) / 64 * 64
 template <typename T, int NMAX> struct MgcLevel {
     static constexpr bool WAVE = NMAX * NMAX <= 64;  // one wave owns the level
     static constexpr int SY = NMAX + 1, SZ = SY * SY;
-    T x[NMAX], b[NMAX];  // b: h^2 times the right-hand side
+    T x[NMAX], b[NMAX];
     T d0, d1, d2;        // the diagonal on the first, the inner and the last plane
     T o0, o1, o2;        // omega / diagonal there
-    T h2, inv_h2, rest;
+    T h2, inv_h2;
     T *c;  // the column's first point in LDS
     int n;
     bool own;
@@ -648,7 +648,6 @@ template <typename T, int NMAX> struct MgcLevel {
         h2 = (T)a.h2[l];
         inv_h2 = T(1) / h2;
         const T omega = (T)a.omega;
-        rest = T(1) - omega;
         c = lds + SZ + 1 + (own ? i + SY * j : 0);
         const T gl = (T)a.gl[l], gh = (T)a.gh[l];
         T g = T(0);
@@ -677,7 +676,7 @@ template <typename T, int NMAX> struct MgcLevel {
     __device__ T around(int k) const { return ((c[SZ * k - 1] + c[SZ * k + 1]) + c[SZ * k - SY]) + c[SZ * k + SY]; }
     __device__ void sweep0() {  // from x = 0
 #pragma unroll
-        for (int k = 0; k < NMAX; k++) x[k] = od(k) * b[k];
+        for (int k = 0; k < NMAX; k++) x[k] = od(k) * (h2 * b[k]);
         put(x);
     }
     __device__ void sweep() {
@@ -685,7 +684,9 @@ template <typename T, int NMAX> struct MgcLevel {
 #pragma unroll
         for (int k = 0; k < NMAX; k++) {
             const T xk = x[k], nb = (around(k) + below) + (k + 1 < NMAX ? x[k + 1] : T(0));
-            x[k] = rest * xk + od(k) * (b[k] + nb);  // x + (omega / d) (h^2 b + nb - d x)
+            // as a correction to x: (1 - omega) x + (omega / d) (h^2 b + nb) rounds at x's size twice, and the f32 cycle's
+            // error against 64 bits was 1.2 to 2.2 times this form's
+            x[k] = xk + od(k) * (h2 * b[k] + (nb - diag(k) * xk));
             below = xk;
             if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // few neighbour reads in flight at once: registers
         }
@@ -696,7 +697,7 @@ template <typename T, int NMAX> struct MgcLevel {
 #pragma unroll
         for (int k = 0; k < NMAX; k++) {
             const T nb = (around(k) + (k > 0 ? x[k - 1] : T(0))) + (k + 1 < NMAX ? x[k + 1] : T(0));
-            r[k] = k < n ? inv_h2 * (b[k] + nb - diag(k) * x[k]) : T(0);
+            r[k] = k < n ? b[k] + inv_h2 * (nb - diag(k) * x[k]) : T(0);
             if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
         }
         put(r);
@@ -717,7 +718,7 @@ template <typename T, int NMAX> struct MgcLevel {
 #pragma unroll
         for (int k = 0; k < NMAX; k++) {
             const T mid = plane(2 * k + 1), hi = plane(2 * k + 2);  // plane NF: the border
-            b[k] = k < n ? h2 * (T(0.25) * (lo + hi) + T(0.5) * mid) : T(0);
+            b[k] = k < n ? T(0.25) * (lo + hi) + T(0.5) * mid : T(0);
             lo = hi;
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -787,7 +788,7 @@ __global__ __launch_bounds__(mgc_threads(NMAX)) void k_mg_coarse(T *x_out, const
 #pragma unroll
     for (int k = 0; k < NMAX; k++) {
         const T v = b_in[at + nn * min(k, n - 1)];
-        L.b[k] = k < n ? L.h2 * v : T(0);
+        L.b[k] = k < n ? v : T(0);
     }
     constexpr int ELEMS = MgcElems<NMAX>::value, THREADS = mgc_threads(NMAX);
     for (int e = threadIdx.x; e < ELEMS; e += THREADS) lds[e] = T(0);

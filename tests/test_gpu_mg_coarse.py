@@ -58,3 +58,56 @@ def test_the_fused_cycle_matches_numpy(n, precision):
     # level to level: 100 roundings
     bound = 100 * (2.0 ** -53 if precision == lira.FP64 else 2.0 ** -24)
     assert np.abs(z - want).max() <= bound * np.abs(want).max()
+
+
+def _cycle_f32(n, h, d_low, d_high, b):
+    """The same cycle with every operation rounded to f32 (the transfers once per point)."""
+    f = np.float32
+    edge = np.zeros(n)
+    edge[0] += 1.0 - 1.0 / d_low
+    edge[-1] += 1.0 - 1.0 / d_high
+    diag = (6.0 - (edge[:, None, None] + edge[None, :, None] + edge[None, None, :])).astype(f)
+    h2, factor = f(h * h), f(OMEGA) / diag
+
+    def defect(x):  # the sum of the neighbours less diag x
+        p = np.pad(x, 1)
+        return (((((p[1:-1, 1:-1, :-2] + p[1:-1, 1:-1, 2:]) + p[1:-1, :-2, 1:-1]) + p[1:-1, 2:, 1:-1])
+                 + p[:-2, 1:-1, 1:-1]) + p[2:, 1:-1, 1:-1]) - diag * x
+
+    def sweeps(x, count):
+        for _ in range(count):
+            x = x + factor * (h2 * b + defect(x))
+        return x
+
+    x = np.zeros_like(b)
+    if n <= 2:
+        return sweeps(x, COARSE)
+    x = sweeps(x, PRE)
+    r = b + defect(x) / h2
+    nc = n // 2
+    w = np.zeros((nc, n))
+    for i in range(nc):
+        for d, v in ((-1, 0.25), (0, 0.5), (1, 0.25)):
+            if 2 * i + 1 + d < n:
+                w[i, 2 * i + 1 + d] = v
+    bc = np.einsum("az,by,cx,zyx->abc", w, w, w, r, optimize=True).astype(f)
+    xc = _cycle_f32(nc, 2.0 * h, (d_low + 1.0) / 2.0, (d_high + (n - 2 * nc)) / 2.0, bc)
+    x = x + np.einsum("az,by,cx,abc->zyx", 2 * w, 2 * w, 2 * w, xc, optimize=True).astype(f)
+    return sweeps(x, POST)
+
+
+@pytest.mark.parametrize("n", [5, 6, 8, 11, 12, 13, 16])
+def test_the_f32_cycle_is_as_accurate_as_its_operations(n):
+    import torch
+    assert torch.cuda.is_available(), "GPU tests need a HIP device"
+    import lira
+    h, solver = 0.3, lira.GpuSolver(n, 0.3, lira.MIXED)
+    ours = rounded = 0.0
+    for seed in range(4):
+        r = np.random.default_rng(10 * n + seed).standard_normal((n, n, n)).astype(np.float32)
+        want = _cycle(n, h, 1.0, 1.0, r.astype(float))
+        got = solver.mg_vcycle(r.astype(float).reshape(-1)).reshape(n, n, n)
+        ours += np.log(np.linalg.norm(got - want))
+        rounded += np.log(np.linalg.norm(_cycle_f32(n, h, 1.0, 1.0, r) - want))
+    # the mean of the logarithms: the kernel's fused operations may only make its error smaller
+    assert ours <= rounded
