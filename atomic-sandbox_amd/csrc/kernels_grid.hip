@@ -81,10 +81,10 @@ template <> __device__ __forceinline__ void bstore_nt<double>(double v, BufRes r
 //   sum_m c_m (f_m - 2 f_0 + f_{-m}) = sum_{j=0..3} K_j (D_j - D_{-1-j}),  K_j = sum_{m>j} c_m.
 // A difference of neighbouring values of a smooth field is exact or nearly so in its own precision, and the sum of
 // second differences never carries the large central term, so the f32 stencil keeps its accuracy (2-norm error of H.X
-// against 64 bits on orbital-like bands, 95^3: 6e-8 .. 8e-8). Neighbouring outputs share their D's: along z they stay in
-// registers (four below the plane, four of the planes ahead), along x a lane's VX points share VX + 7, and each axis costs 8 more operations per
-// point: 41 VALU operations per f32 point, against 56 of the pair form c_m [(f_m - f_0) + (f_{-m} - f_0)] that this
-// replaces. Without packed FP32 instructions an f32 operation issues at the f64 rate (39 T lane-operations/s), so at
+// against 64 bits on orbital-like bands, 95^3: 4e-8 .. 7e-8). Neighbouring outputs share their D's: along z they stay in
+// registers (four below the plane, four of the planes ahead), along x a lane's VX points share VX + 7, and each axis
+// costs 8 more operations per point: 41 VALU operations per f32 point, against 56 of the pair form c_m [(f_m - f_0) +
+// (f_{-m} - f_0)] that this replaces. Without packed FP32 instructions an f32 operation issues at the f64 rate (39 T lane-operations/s), so at
 // 192^3 x 64 the pair form alone cost 0.65 ms of VALU issue against 0.63 ms for the bytes at the copy rate.
 //
 // XCD-aware workgroup order. The dispatcher hands consecutive workgroup ids to the 8 XCDs round-robin (id mod 8);
@@ -171,8 +171,9 @@ template <> struct StK<float> {
 // z + 6), D the differences D_{z-4} .. D_{z-1} (D_j in slot (j - z0) mod 4; step z replaces D_{z-4} by D_z), and hq /
 // vq / rq its halo vectors, V and R, loaded two planes ahead. The z loop is unrolled by 8 so every slot is a compile-time
 // constant: registers rotate by name, and a load is only waited for when its plane is used. Keeping D_z .. D_{z+3} as
-// well would save three operations per point but 16 registers: at three waves per SIMD (168 registers) the Jacobi sweep
-// then spills (95^3 x 8 f32: 24.9 us, 19.6 us without them).
+// well would save three operations per point but 16 registers: at three waves per SIMD (168 registers) the f32 Jacobi
+// sweep then spills (95^3 x 8: 24.9 us, 19.6 us without them). The f64 sweep on rows that are no whole vectors is past
+// that limit as it is, by 7 or 8 registers.
 template <typename T, int HV> struct StRegs {
     typedef typename Vec16<T>::type V;
     V F[8], D[4];
@@ -491,8 +492,10 @@ static int st_chunk(int tx, int n, int nb, int esize) {
 }
 
 // The tile when no tuned choice exists: the narrowest one that takes whole rows up to 128 points (no x halos), in f32
-// also 192-wide rows that fill it; 64-wide otherwise; in balanced chunks. Over 66 shapes (25^3 .. 256^3, 1 .. 32 bands,
-// three modes, both types) its time was within 3 % of the best variant's in the geometric mean.
+// also 192-wide rows that fill it; 64-wide otherwise; in balanced chunks. Over 72 shapes (25^3 .. 256^3, 1 .. 64 bands,
+// three modes, both types) its time was 1.03 of the best variant's in the geometric mean, and on single shapes up to 1.24
+// (72^3 x 10 f64; 40^3 x 24 f64 1.16, 176^3 x 4 f32 1.14, 64^3 x 32 f32 1.13, 160^3 x 12 f32 1.10): the solver, and a
+// caller of lira_autotune_stencil, time the variants on their own shape.
 static int pick_variant(int n, int esize) {
     const int tx = n <= 64 ? 64 : n <= 96 ? 96 : n <= 128 ? 128 : esize == 4 && n > 176 && n <= 192 ? 192 : 64;
     for (int v = 0; v < stencil_variants(); v++)

@@ -447,7 +447,8 @@ static void wait_event(hipEvent_t e) {
 // use): each worker has two slots, and copies one while the link moves the other. One thread copies 28 GB/s and less
 // where it touches new pages, so large fields take four workers; below 16 MiB starting threads costs more than they
 // save. On the Poisson problem of 256^3 (402 MB of transfers) a call went from 31.1 to 20.4 ms, at 95^3 (21 MB) from
-// 3.61 to 3.47 ms. One transfer at a time, as the solver's stream and fields are.
+// 3.61 to 3.47 ms; a solver's first call, which pins the slots, from 35 to 30-34 and from 5.8 to 4.0 ms. One transfer at a
+// time, as the solver's stream and fields are.
 class HostStage {
     static constexpr size_t SLOT = (size_t)2 << 20, THREADED = (size_t)16 << 20;
     static constexpr int WORKERS = 4, SLOTS = 2;
