@@ -30,7 +30,7 @@ void DevBuf::release() {
 }
 
 // 8th-order second-derivative coefficients c1..c4 (qm/src/stencil.rs:24), c0 = -205/72 = -2 sum c_m. The kernels use
-// their partial sums in their own precision (StK below): a bare double constant would promote an f32 stencil's products
+// their partial sums in their own precision (StCoef below): a bare double constant would promote an f32 stencil's products
 // to f64.
 #define C1 (8.0 / 5.0)
 #define C2 (-1.0 / 5.0)
@@ -48,8 +48,12 @@ void DevBuf::release() {
 constexpr unsigned BUF_OOB = 0x80000000u;
 typedef __amdgpu_buffer_rsrc_t BufRes;
 __device__ __forceinline__ BufRes field_res(const void *base, long bytes) {
-    // word 3 = 0x00020000: 32-bit data format, no swizzle, raw addressing (the gfx9 family's value)
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, (int)bytes, 0x00020000);
+    // word 3 = 0x00020000: 32-bit data format, no swizzle, raw addressing (the gfx9 family's value). Opaque to the compiler,
+    // so that each descriptor keeps its four registers: it shared the equal words 2 and 3 of a kernel's descriptors and
+    // moved them at every use (95^3 x 16 f32 31.4 us, 31.0 without).
+    int range = (int)bytes, format = 0x00020000;
+    asm volatile("" : "+s"(range), "+s"(format));
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, range, format);
 }
 __device__ __forceinline__ unsigned row_off(int xx, int yy, int n, int esize) {
     return (xx >= 0 && xx < n && yy >= 0 && yy < n) ? (unsigned)(xx + n * yy) * (unsigned)esize : BUF_OOB;
@@ -155,17 +159,25 @@ template <typename V> __device__ __forceinline__ void bstorev_nt(V v, BufRes r, 
 }
 
 constexpr int ST_AHEAD = 6;  // a lane loads its plane z + ST_AHEAD at plane z
-// K_j = sum_{m > j} c_m. Rounded to f32 one by one they would scale every Laplacian by 1 + 5.3e-8 (sum (2j + 1) K_j, K_0's
-// rounding); the f32 set takes the neighbouring values (2, 4 and 8 units in the last place off) that keep that sum within
-// 6e-9 of 1 and the 4th moment within 6e-8 of 0.
-template <typename T> struct StK;
-template <> struct StK<double> {
-    static constexpr double k[4] = {C1 + C2 + C3 + C4, C2 + C3 + C4, C3 + C4, C4};
+// factor K_j, K_j = sum_{m > j} c_m, in the kernel's precision; factor is -1/2 / h^2, or scale / h^2. A sum (2j + 1) k_j
+// that is off by d scales every kinetic energy by 1 + d, so a total energy is off by d times it, and in f32 the k_j rounded
+// one by one give d up to 1e-7. k_0 and k_1 are rounded; k_2 and k_3 are small, so finely spaced in f32, and make up what
+// these lost in that sum and in the 4th moment: d is below 1e-9, the 4th moment's error below 1e-8.
+template <typename T> struct StCoef {
+    T k[4];
 };
-template <> struct StK<float> {
-    static constexpr float k[4] = {1.4236111640930176f, -0.1763889193534851f, 0.023611119017004967f,
-                                   -0.0017857152270153165f};
-};
+template <typename T> static StCoef<T> st_coef(double factor) {
+    const double K[4] = {factor * (C1 + C2 + C3 + C4), factor * (C2 + C3 + C4), factor * (C3 + C4), factor * C4};
+    StCoef<T> c;
+    for (int j = 0; j < 4; j++) c.k[j] = (T)K[j];
+    if (!std::isfinite(c.k[0])) return c;
+    const double e0 = K[0] - (double)c.k[0], e1 = K[1] - (double)c.k[1];
+    const double m2 = e0 + 3.0 * e1, m4 = e0 + 15.0 * e1;  // (j + 1)^p - j^p: 1, 3, 5, 7 and 1, 15, 65, 175
+    const double x3 = (m4 - 13.0 * m2) / 84.0, x2 = (m2 - 7.0 * x3) / 5.0;
+    c.k[2] = (T)(K[2] + x2);
+    c.k[3] = (T)(K[3] + (m2 + 5.0 * (K[2] - (double)c.k[2])) / 7.0);
+    return c;
+}
 
 // Register state of a lane: F holds its vector on planes z .. z + 5 (plane p in slot (p - z0) mod 8; step z loads plane
 // z + 6), D the differences D_{z-4} .. D_{z-1} (D_j in slot (j - z0) mod 4; step z replaces D_{z-4} by D_z), and hq /
@@ -192,7 +204,8 @@ template <typename T, int HV> struct StCtx {
     int nv;                 // points of the lane's vector inside the box
     int lo;                 // the lane's element offset in an LDS plane
     int n, zlim;            // planes at or past zlim are not loaded
-    T hs, omega, diag_t, lamb;
+    StCoef<T> cf;
+    T omega, diag_t, lamb;
     // plane zz at byte offset off; a plane past the last one the chunk needs reads plane n: out of range, 0
     __device__ V ld(BufRes r, unsigned off, int zz, int lim) const {
         return bloadv<T>(r, off + (unsigned)(zz < lim ? zz : n) * pb);
@@ -243,9 +256,9 @@ __device__ __forceinline__ void st_plane(StRegs<T, HV> &R, const StCtx<T, HV> &c
         V dn[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) dn[j] = R.F[(S + j + 1) & 7] - R.F[(S + j) & 7];
-        acc = (dn[3] - R.D[S & 3]) * StK<T>::k[3];
-        add(dn[2] - R.D[(S + 1) & 3], StK<T>::k[2]);
-        add(dn[1] - R.D[(S + 2) & 3], StK<T>::k[1]);
+        acc = (dn[3] - R.D[S & 3]) * c.cf.k[3];
+        add(dn[2] - R.D[(S + 1) & 3], c.cf.k[2]);
+        add(dn[1] - R.D[(S + 2) & 3], c.cf.k[1]);
         e0 = dn[0] - R.D[(S + 3) & 3];
         R.D[S & 3] = dn[0];
     }
@@ -258,9 +271,9 @@ __device__ __forceinline__ void st_plane(StRegs<T, HV> &R, const StCtx<T, HV> &c
             m[q] = *reinterpret_cast<const V *>(tl + c.lo - q * LXP);
             p[q] = *reinterpret_cast<const V *>(tl + c.lo + q * LXP);
         }
-        add((p[4] - p[3]) - (m[3] - m[4]), StK<T>::k[3]);
-        add((p[3] - p[2]) - (m[2] - m[3]), StK<T>::k[2]);
-        add((p[2] - p[1]) - (m[1] - m[2]), StK<T>::k[1]);
+        add((p[4] - p[3]) - (m[3] - m[4]), c.cf.k[3]);
+        add((p[3] - p[2]) - (m[2] - m[3]), c.cf.k[2]);
+        add((p[2] - p[1]) - (m[1] - m[2]), c.cf.k[1]);
         e0 += (p[1] - p[0]) - (m[0] - m[1]);
     }
     // x: the VX + 8 points of this row about the lane's, their differences shared by its points
@@ -283,11 +296,11 @@ __device__ __forceinline__ void st_plane(StRegs<T, HV> &R, const StCtx<T, HV> &c
 #pragma unroll
         for (int j = 3; j >= 1; j--)
 #pragma unroll
-            for (int i = 0; i < VX; i++) acc[i] = st_fma(d[4 + i + j] - d[3 + i - j], StK<T>::k[j], acc[i]);
+            for (int i = 0; i < VX; i++) acc[i] = st_fma(d[4 + i + j] - d[3 + i - j], c.cf.k[j], acc[i]);
 #pragma unroll
         for (int i = 0; i < VX; i++) e0[i] += d[4 + i] - d[3 + i];
     }
-    add(e0, StK<T>::k[0]);
+    add(e0, c.cf.k[0]);
     // the kinetic term is rounded and the potential's product is not: near the nuclei the two nearly cancel, and the product
     // is the larger one (f32 error of H.X against 64 bits over 40 drawn fields, to that of the pair form c_m [(f_m - f_0) +
     // (f_{-m} - f_0)]: 0.73 .. 1.00 of it, 0.87 in the mean; with the product rounded instead up to 1.4)
@@ -295,12 +308,12 @@ __device__ __forceinline__ void st_plane(StRegs<T, HV> &R, const StCtx<T, HV> &c
 #pragma unroll
     for (int i = 0; i < VX; i++) {
         if (MODE == ST_LAP) {
-            o[i] = c.hs * acc[i];
+            o[i] = acc[i];
         } else if (MODE == ST_HAM) {
-            o[i] = st_fma(R.vq[S & 1][i], ce[i], c.hs * acc[i]);
+            o[i] = st_fma(R.vq[S & 1][i], ce[i], acc[i]);
         } else {
             const T t = R.vq[S & 1][i] - c.lamb;
-            const T hw = st_fma(t, ce[i], c.hs * acc[i]);
+            const T hw = st_fma(t, ce[i], acc[i]);
             T d = c.diag_t + t;
             d = d > T(0.1) ? d : T(0.1);
             o[i] = st_fma(st_quot(c.omega, d), R.rq[S & 1][i] - hw, ce[i]);
@@ -326,7 +339,7 @@ template <typename T, int MODE, int TXL, int TYL, bool XT, bool RAG>
 __global__ __launch_bounds__(TXL *TYL) __attribute__((amdgpu_waves_per_eu(3))) void k_stencil(const T *__restrict__ x, T *__restrict__ out,
                                                       const T *__restrict__ v, const T *__restrict__ r,
                                                       const double *__restrict__ lam, int n, long N, int zc, int nb,
-                                                      int order, T hs, T omega, T diag_t, const T *__restrict__ x2,
+                                                      int order, StCoef<T> cf, T omega, T diag_t, const T *__restrict__ x2,
                                                       T *__restrict__ out2, int nb1) {
     typedef typename Vec16<T>::type V;
     constexpr int VX = Vec16<T>::N, TX = TXL * VX, LXP = TX + 8, THREADS = TXL * TYL;
@@ -354,7 +367,7 @@ __global__ __launch_bounds__(TXL *TYL) __attribute__((amdgpu_waves_per_eu(3))) v
     c.co = row_off(gx, y0 + ty, n, (int)sizeof(T));
     c.nv = n - gx;
     c.lo = (ty + 4) * LXP + 4 + VX * tx;
-    c.hs = hs;
+    c.cf = cf;
     c.omega = omega;
     c.diag_t = diag_t;
     // halo vectors: the 4 rows above and below the tile, then (XT) each row's 4 points left and right of it
@@ -514,11 +527,11 @@ static void launch_stencil(const StencilParams &p, int zc, int order, const T *x
     const int nzc = (n + zc - 1) / zc;
     const dim3 grid(st_grid((n + TX - 1) / TX, (n + TYL - 1) / TYL, nzc, p.nb, order)), block(TXL * TYL);
     const double inv_h2 = 1.0 / (p.h * p.h);
-    const T hs = (T)(MODE == ST_LAP ? p.scale * inv_h2 : -0.5 * inv_h2);
+    const StCoef<T> cf = st_coef<T>(MODE == ST_LAP ? p.scale * inv_h2 : -0.5 * inv_h2);
     const int nb1 = p.nb1 < 0 ? p.nb : p.nb1;
 #define LIRA_GO(RAG_)                                                                                                   \
     hipLaunchKernelGGL((k_stencil<T, MODE, TXL, TYL, XT, RAG_>), grid, block, 0, s, x, out, v, r, lam, n, N, zc, p.nb, \
-                       order, hs, (T)p.omega, (T)p.diag_t, static_cast<const T *>(p.x2), static_cast<T *>(p.out2), nb1)
+                       order, cf, (T)p.omega, (T)p.diag_t, static_cast<const T *>(p.x2), static_cast<T *>(p.out2), nb1)
     if (n % VX) LIRA_GO(true);
     else LIRA_GO(false);
 #undef LIRA_GO

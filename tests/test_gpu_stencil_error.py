@@ -65,3 +65,25 @@ def test_the_error_is_no_larger_than_the_pair_forms(n, h):
         ours += np.log(np.linalg.norm(out.cpu().numpy().reshape(n, n, n) - want) / size)
         pair += np.log(np.linalg.norm(_pair_form(x, v, h) - want) / size)
     assert ours <= pair  # the mean over the fields, of the logarithm of the relative error
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("h", [0.07, 0.12, 0.15, 0.2, 0.25, 0.3, 0.35])
+def test_the_kinetic_energy_has_no_common_factor(h):
+    # A smooth field's f32 -1/2 lap is that of 64 bits times 1 + d. Each point's rounding, 2^-24, averages out of d over some
+    # 1100 points (by weight) to 1.8e-9, over three fields to 1e-9; the fields are 1e-6 of their peak at the faces.
+    import torch
+    assert torch.cuda.is_available(), "GPU tests need a HIP device"
+    import lira
+    n, d = 64, []
+    a = (np.arange(n) - (n - 1) / 2) / n
+    for seed in range(3):
+        rng = np.random.default_rng(seed)
+        p, w = rng.uniform(-0.05, 0.05, 3), rng.uniform(55, 75, 3)
+        x = np.exp(-w[0] * (a[:, None, None] - p[0]) ** 2 - w[1] * (a[:, None] - p[1]) ** 2 - w[2] * (a - p[2]) ** 2).astype(F)
+        want = _exact(x, np.zeros_like(x), h)
+        out = torch.empty(1, n ** 3, dtype=torch.float32, device="cuda")
+        lira.hamiltonian(n, h, torch.zeros(n ** 3, device="cuda"), torch.from_numpy(x.reshape(1, -1).copy()).cuda(), out, 1)
+        got = out.cpu().numpy().reshape(n, n, n).astype(float)
+        d.append((got * want).sum() / (want * want).sum() - 1.0)
+    assert abs(np.mean(d)) < 3e-9
