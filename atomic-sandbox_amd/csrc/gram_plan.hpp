@@ -16,7 +16,8 @@ constexpr int gram_computed(int RB, int CB, bool SHARE) { return RB * CB - (SHAR
 constexpr int gram_waves(int RB, int CB, bool SHARE) { return !SHARE ? 4 : RB * CB <= 6 && CB <= 3 ? 16 : 8; }
 // whether the accumulators and `each` registers a loaded block fit what the waves leave a lane, 128 or 256
 constexpr bool gram_fits(int RB, int CB, bool SHARE, int each) {
-    return 8 * gram_computed(RB, CB, SHARE) + each * gram_loaded(RB, CB, SHARE) <= (gram_waves(RB, CB, SHARE) == 16 ? 124 : 240);
+    return 8 * gram_computed(RB, CB, SHARE) + each * gram_loaded(RB, CB, SHARE) <=
+           (gram_waves(RB, CB, SHARE) == 16 ? 124 : 240);
 }
 // How a lane loads a 16-column block (GramLoad in kernels_grid.hip). QUAD: four consecutive points of one column. PAIR: 16
 // bytes of each of two columns, so that a load instruction takes 128 bytes of a column instead of 64; it needs two column
@@ -36,9 +37,9 @@ constexpr int gram_unit(int depth, int esize, int loads) { return depth * (loads
 // The tiling of an m x q product: nr x nc tiles of RB x CB 16 x 16 blocks (the blocks split evenly, at most 3 x 6 in f32
 // or where the one tile shares its operands, else 3 x 4: the accumulators and two units of operands fill 256 registers. In
 // f32 without sharing 3 x 6 spills 69 more, and reads each column fewer times: 138 x 276 on 160^3 5.70 ms, 6.32 with 3 x 4;
-// 96 x 192 on 95^3 533 us and 509) and the chunks of points. A product of one shared tile takes one workgroup per CU, 16 waves (4 per SIMD, up to 128
-// registers) or 8; several tiles take two 4-wave workgroups per CU, so that the tiles that S^T S's symmetry empties or
-// thins leave room for others. The partials of one product stay within GRAM_PARTIALS doubles (lira_gram_noalloc's fixed
+// 96 x 192 on 95^3 533 us and 509) and the chunks of points. A product of one shared tile takes one workgroup per CU, 16
+// waves (4 per SIMD, up to 128 registers) or 8; several tiles take two 4-wave workgroups per CU, so that the tiles that
+// S^T S's symmetry empties or thins leave room for others. The partials of one product stay within GRAM_PARTIALS doubles (lira_gram_noalloc's fixed
 // array) whenever one chunk's do.
 struct GramPlan {
     int RB, CB, nr, nc, chunks, loads;
@@ -58,9 +59,9 @@ inline GramPlan gram_plan(int m, int q, long N, int esize, bool sym) {
     g.nc = (C + most - 1) / most;
     g.CB = (C + g.nc - 1) / g.nc;
     g.nc = (C + g.CB - 1) / g.CB;
-    // PAIR, where it fits, in f64 for more columns than the 256 MiB cache holds (24 x 48 on 95^3 86 -> 75 us, on 64^3 20 -> 22),
-    // in f32 for more than 32 columns a multiple of 8 MiB apart; one block of columns (f64) or two (f32) gained nothing.
-    // PAIR2 in f64 from 185^3 on. GramLoad has both sides.
+    // PAIR, where it fits, in f64 for more columns than the 256 MiB cache holds (24 x 48 on 95^3 86 -> 75 us; 16 x 32 on
+    // 64^3 20 -> 22), in f32 for more than 32 columns a multiple of 8 MiB apart; one block of columns (f64) or two (f32)
+    // gained nothing. PAIR2 in f64 from 185^3 on. GramLoad has both sides.
     g.loads = GRAM_QUAD;
     if (gram_has(g.RB, g.CB, g.share, esize, GRAM_PAIR) &&
         (esize == 8 ? g.CB > 1 && q * N * 8 >= 256L << 20 : g.CB > 2 && N * 4 % (8L << 20) == 0))

@@ -88,8 +88,9 @@ template <> __device__ __forceinline__ void bstore_nt<double>(double v, BufRes r
 // against 64 bits on orbital-like bands, 95^3: 4e-8 .. 7e-8). Neighbouring outputs share their D's: along z they stay in
 // registers (four below the plane, four of the planes ahead), along x a lane's VX points share VX + 7, and each axis
 // costs 8 more operations per point: 40 VALU operations per f32 point, against 56 of the pair form c_m [(f_m - f_0) +
-// (f_{-m} - f_0)] that this replaces. Without packed FP32 instructions an f32 operation issues at the f64 rate (39 T lane-operations/s), so at
-// 192^3 x 64 the pair form alone cost 0.65 ms of VALU issue against 0.63 ms for the bytes at the copy rate.
+// (f_{-m} - f_0)] that this replaces. Without packed FP32 instructions an f32 operation issues at the f64 rate (39 T
+// lane-operations/s), so at 192^3 x 64 the pair form alone cost 0.65 ms of VALU issue against 0.63 ms for the bytes at the
+// copy rate.
 //
 // XCD-aware workgroup order. The dispatcher hands consecutive workgroup ids to the 8 XCDs round-robin (id mod 8);
 // each XCD has its own L2. The stencil launches a 1-D grid and gives XCD x the contiguous logical range
